@@ -63,7 +63,7 @@ constexpr double kNoEnd = 1.0e300; // end time of a model advanced by or_model_r
 constexpr int kVariants = 4;
 constexpr int kTile = orasm::kTile;
 static_assert(kTile == kBlock, "element tiles and node blocks share the workgroup size");
-template <typename R> constexpr int variant_waves(int v) { return 2 + (v & 1); }
+template <typename R> constexpr int variant_waves(int v) { return sizeof(R) == 8 ? 2 : 2 + (v & 1); }
 
 // MSTOP codes (include/or_gpu.h): an element's non-positive Jacobian, a time step <= 0
 constexpr int32_t kMstopJacobian = 1, kMstopTimeStep = 2;
@@ -103,6 +103,7 @@ __device__ __forceinline__ int64_t xcd_contiguous_block(int64_t b, int64_t nb) {
 // though the kernels read them from a descriptor in memory.
 template <typename T> using gptr = __attribute__((address_space(1))) T *;
 typedef double v2d __attribute__((ext_vector_type(2))); // 16-byte load / store unit
+template <typename T> using cptr = const __attribute__((address_space(4))) T *; // read-only: scalar loads
 template <typename T> __device__ __forceinline__ gptr<T> to_global(T *p) { return (gptr<T>)p; }
 template <typename T> __device__ __forceinline__ gptr<T> to_global(const void *p) { return (gptr<T>)(T *)p; }
 
@@ -257,14 +258,19 @@ template <typename S, int W, int NK> struct TileAssembly {
   int32_t j, j1, node;
   v4u src;
 
+  // The tile's range of the prefix list, read at the kernel's start (uniform: scalar loads),
+  // so that prefetch needs no load before its own.
+  __device__ __forceinline__ void range(const int32_t *fr_start, int64_t tile) {
+    const cptr<int32_t> p = (cptr<int32_t>)(fr_start + tile);
+    j = p[0] + (int32_t)threadIdx.x;
+    j1 = p[1];
+  }
+
   __device__ __forceinline__ void prefetch(gptr<const int32_t> restp, int64_t ne, int64_t i,
-                                           gptr<const int32_t> fr_start, gptr<const int32_t> fr_node,
-                                           gptr<const v4u> fr_src, int64_t tile) {
-    __asm__ __volatile__("" ::: "memory"); // after the element chain, not hoisted into it
+                                           gptr<const int32_t> fr_node, gptr<const v4u> fr_src) {
+    __asm__ __volatile__("" ::: "memory"); // where the caller puts it, not hoisted
 #pragma unroll
     for (int k = 0; k < NK; ++k) rest[k] = (i < ne) ? restp[(int64_t)k * ne + i] : -1;
-    j = fr_start[tile] + (int32_t)threadIdx.x;
-    j1 = fr_start[tile + 1];
     if (j < j1) {
       node = fr_node[j];
       src = fr_src[j];
@@ -344,49 +350,91 @@ template <int TB, typename R> __device__ __forceinline__ void tile_ehou_commit(c
   }
 }
 
-// ---------------------------------------------------------------- hex element kernel
-// In the split form, the hex element state read by the material phase (SIG(6), EINT, RHO,
-// VOL0, PLA, EPSD, QVIS) is copied from HBM to LDS by the wave itself at the start of the chain, with
-// global-to-LDS loads that occupy no registers: the copy is in flight during the gather,
-// the geometry and the kinematics, and the material phase reads LDS.  Word a of the
-// tile's element t sits at sst[a * kTile + t]; each wave copies its own 64 elements, so
-// only the wave's own wait for its loads orders the copy before its reads.
-constexpr int kHexStagedWords = 12;
+// ---------------------------------------------------------------- element state in LDS
+// The element state that the hex chain's material phase reads (SIG(6), EINT, RHO, VOL0, PLA, EPSD,
+// QVIS) is copied from HBM to LDS by the wave itself at the start of the chain, with
+// global-to-LDS loads that occupy no registers: the copy is in flight during the gather and the
+// geometry.  It uses the LDS words in which the same threads leave their force rows at the
+// chain's end (24 words per element):
+// word a of the tile's element t sits at lds[a * kTile + t], and each wave copies and reads
+// its own 64 elements only, so the wave's own wait for its loads orders the copy before its reads
+// and its reads precede its writes of the rows.
 typedef __attribute__((address_space(3))) void *lds_void;
+typedef __attribute__((address_space(3))) char *lds_char;
 
+// One state word (src) of the wave's 64 elements into word a of the tile's LDS.
 template <typename S>
-__device__ __forceinline__ void stage_hex_state(S *sst, const HexPtrs<S> &e, int64_t first) {
+__device__ __forceinline__ void stage_word(S *lds, int a, gptr<const S> src, int64_t first, int64_t ne) {
   constexpr int D = sizeof(S) / 4; // dwords per word
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t wfirst = first + 64 * w;
-  const gptr<const S> src[kHexStagedWords] = {e.sig,          e.sig + e.ne,     e.sig + 2 * e.ne, e.sig + 3 * e.ne,
-                                              e.sig + 4 * e.ne, e.sig + 5 * e.ne, e.eint,           e.rho,
-                                              e.vol0,         e.pla,            e.epsd,           e.qvis};
 #pragma unroll
-  for (int a = 0; a < kHexStagedWords; ++a) {
-#pragma unroll
-    for (int h = 0; h < D; ++h) {
-      const int d = h * 64 + l; // dword of the wave's slice
-      if (wfirst + d / D < e.ne)
-        __builtin_amdgcn_global_load_lds((gptr<void>)((gptr<const char>)(src[a] + wfirst) + 4 * d),
-                                         (lds_void)((char *)(sst + a * kTile + 64 * w) + 256 * h), 4, 0, 0);
-    }
+  for (int h = 0; h < D; ++h) {
+    const int d = h * 64 + l; // dword of the wave's slice
+    if (wfirst + d / D < ne)
+      __builtin_amdgcn_global_load_lds((gptr<void>)((gptr<const char>)(src + wfirst) + 4 * d),
+                                       (lds_void)((char *)(lds + a * kTile + 64 * w) + 256 * h), 4, 0, 0);
   }
 }
 
 // The wave's global-to-LDS loads have landed (they count as vector memory loads).
 __device__ __forceinline__ void wait_staged() { __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-template <typename R, typename S, int TB, int W, bool EH>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_hex_forces(
-    const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int parity_output) {
-  static_assert(TB == kTile, "a hex workgroup is one assembly tile");
+// The tables of or_math.h in LDS, one copy for each wave, read from memory when the wave first
+// needs them.  A look-up in memory costs a wave 500-600 clocks, and a plastic shell point makes
+// ten in one chain: the tube of 72,000 shells, deep in plasticity, takes 38 us instead of 42.
+// A wave without a plastic point reads no table (read at the start by every workgroup, they
+// cost an elastic plate of 2,304 shells 0.5 us of 16.7).
+__device__ __align__(256) constexpr ormath::MathTab kMathTab = ormath::make_math_tab();
+struct WaveTab {
+  const __attribute__((address_space(3))) double *t;
+  bool have; // the same in every lane
+  __device__ __forceinline__ explicit WaveTab(double *copies)
+      : t((const __attribute__((address_space(3))) double *)(copies +
+                                                            ormath::kTabWords * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6))),
+        have(false) {}
+  // Called by whole waves: the copy is read by all lanes when any of them needs it.
+  __device__ __forceinline__ void need(bool cond) {
+    if (have || !__any(cond)) return;
+    constexpr int kBytes = (int)sizeof(ormath::MathTab);
+    static_assert(kBytes % 16 == 0, "16-byte loads");
+    const int l = 16 * (threadIdx.x & 63);
+    const gptr<const char> src = (gptr<const char>)(gptr<const void>)(const void *)&kMathTab;
+#pragma unroll
+    for (int o = 0; o < kBytes; o += 1024)
+      if (o + l < kBytes) __builtin_amdgcn_global_load_lds((gptr<void>)(src + o + l), (lds_void)((lds_char)t + o), 16, 0, 0);
+    wait_staged();
+    have = true;
+  }
+  __device__ __forceinline__ double lg(int i, int k) const { return t[3 * i + k]; }
+  __device__ __forceinline__ double ex(int j, int k) const { return t[ormath::kLogWords + 2 * j + k]; }
+};
+
+// The tables that a shell chain of type R reads (the split form has none).
+template <typename R> __device__ __forceinline__ auto chain_tab(double *copies) {
+  if constexpr (sizeof(R) == 8) return WaveTab(copies);
+  else return ormath::GlobalTab{};
+}
+
+// A tile's LDS: the rows (and the staged state before them), the waves' tables (FP64 shells),
+// EHOU per element.
+template <typename R, typename S, bool EH, bool TAB> struct TileLds {
+  alignas(16) S rows[24 * kTile];
+  alignas(16) double tab[TAB ? kTile / 64 * ormath::kTabWords : 1];
+  double red[kTile / 64];
+  R seh[EH ? kTile : 1];
+};
+static_assert(8 * kHexRowWords == 24 && 4 * kQ4RowWords == 24, "both families keep 24 row words per element");
+
+// ---------------------------------------------------------------- hex element tile
+// The SFORC3 chain of one tile.  Threads past the last element run on the last element's
+// nodes and store nothing, so that the whole workgroup reaches its barriers.
+template <typename R, typename S, bool EH>
+__device__ __forceinline__ void hex_tile(const ModelDev &M, int64_t first, int parity_output,
+                                         TileLds<R, S, EH, false> &sh) {
   // bit 0: cycle parity; bit 1: an output cycle (each element's time-step candidate is kept)
   const int parity = parity_output & 1;
   const bool output = (parity_output & 2) != 0;
-  __shared__ S lds[8 * kHexRowWords * kTile];
-  const Tile tl = tiles[xcd_contiguous_block(blockIdx.x, gridDim.x)];
-  const ModelDev &M = md[tl.model];
   const DevTime *ts = M.ts;
   // a stopped model computes but stores nothing; the flag is tested only before the
   // stores, so that its load overlaps the element's own loads
@@ -394,101 +442,135 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_
   const HexPtrs<S> e = hex_ptrs<S>(M);
   const gptr<const double> xv = to_global<const double>(M.nd.xv);
   const HexConsts &c = M.hc;
-  const int64_t i = (int64_t)tl.first + threadIdx.x;
-  double dtx = kEP06;
-  int mstop = 0;
-  __shared__ R seh[EH ? TB : 1];
+  const int64_t i = first + threadIdx.x;
+  const bool active = i < e.ne;
+  const int64_t ic = active ? i : e.ne - 1;
+  // node ids first (vector loads return in order, and the gather waits for these), then the
+  // copies to LDS, in flight with the gather
   // the split form stages its element state through LDS; the FP64 chain, bound by its
-  // arithmetic at two waves per SIMD, reads it from HBM after the kinematics
+  // arithmetic at two waves per SIMD, reads it from HBM after the kinematics (staged, it took
+  // 15.2 us against 14.5 at 32,000 elements, and the same at 512,000)
   constexpr bool kStage = sizeof(S) == 4;
-  __shared__ S sst[kStage ? kHexStagedWords * kTile : 1];
-  if constexpr (kStage) stage_hex_state<S>(sst, e, tl.first);
-  if (i < e.ne) {
-    const R DT1 = R(time_dt2(ts + parity));
-    HexState<S> st;
-    HexOut<R> o;
-    // EH: the model keeps EHOUR (its own instantiation, so that the other keeps its registers)
-    auto ehou_sink = [&](R v) {
-      if constexpr (EH) seh[threadIdx.x] = v;
+  int32_t nc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) nc[k] = e.conn[(int64_t)k * e.ne + ic];
+  __asm__ __volatile__("" ::: "memory");
+  if constexpr (kStage) {
+    const gptr<const S> src[12] = {e.sig,          e.sig + e.ne,     e.sig + 2 * e.ne, e.sig + 3 * e.ne,
+                                   e.sig + 4 * e.ne, e.sig + 5 * e.ne, e.eint,           e.rho,
+                                   e.vol0,         e.pla,            e.epsd,           e.qvis};
+#pragma unroll
+    for (int a = 0; a < 12; ++a) stage_word<S>(sh.rows, a, src[a], first, e.ne);
+  }
+  TileAssembly<S, kHexRowWords, 8> ta;
+  ta.range(M.hfr_start, first / kTile);
+  const R DT1 = R(time_dt2(ts + parity));
+  HexState<S> st;
+  HexOut<R> o;
+  // EH: the model keeps EHOUR (its own instantiation, so that the other keeps its registers)
+  auto ehou_sink = [&](R v) {
+    if constexpr (EH) sh.seh[threadIdx.x] = v;
+  };
+  double xd[8], yd[8], zd[8];
+  R vx[8], vy[8], vz[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    double a, b, cc, u, v, w;
+    load_node(xv, nc[k], a, b, cc, u, v, w);
+    xd[k] = a; yd[k] = b; zd[k] = cc;
+    vx[k] = R(u); vy[k] = R(v); vz[k] = R(w);
+  }
+  // GBUF%OFF enters the geometry; the rest of the element state is read after the kinematics
+  st.offg = e.offg[ic];
+  auto load_rest = [&]() {
+    if constexpr (kStage) {
+      wait_staged();
+      const S *s = sh.rows + threadIdx.x;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) st.sig[k] = s[k * kTile];
+      st.eint = s[6 * kTile]; st.rho = s[7 * kTile]; st.vol0 = s[8 * kTile]; st.pla = s[9 * kTile];
+      st.epsd = s[10 * kTile]; st.qvis = s[11 * kTile];
+    } else {
+      __asm__ __volatile__("" ::: "memory");
+#pragma unroll
+      for (int k = 0; k < 6; ++k) st.sig[k] = e.sig[(int64_t)k * e.ne + ic];
+      st.eint = e.eint[ic]; st.rho = e.rho[ic]; st.vol0 = e.vol0[ic]; st.pla = e.pla[ic];
+      st.epsd = e.epsd[ic]; st.qvis = e.qvis[ic];
+    }
+  };
+  if constexpr (sizeof(R) == 8) {
+    // FP64: each node's force triple leaves for LDS as soon as it is final, which keeps
+    // the chain within two waves' register budget
+    auto write_row = [&](int k, R fx, R fy, R fz) {
+      const S w[3] = {S(fx), S(fy), S(fz)};
+      lds_corner<S, 3>(sh.rows, k, w);
     };
-    double xd[8], yd[8], zd[8];
-    R vx[8], vy[8], vz[8];
+    hex_element<R, S>(xd, yd, zd, vx, vy, vz, st, c, DT1, o, write_row, load_rest, ehou_sink);
+  } else {
+    // FP32: the forces are gathered first and stored together (registers are not the limit)
+    R f1[8], f2[8], f3[8];
+    auto keep = [&](int k, R fx, R fy, R fz) { f1[k] = fx; f2[k] = fy; f3[k] = fz; };
+    hex_element<R, S>(xd, yd, zd, vx, vy, vz, st, c, DT1, o, keep, load_rest, ehou_sink);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      double a, b, cc, u, v, w;
-      load_node(xv, e.conn[(int64_t)k * e.ne + i], a, b, cc, u, v, w);
-      xd[k] = a; yd[k] = b; zd[k] = cc;
-      vx[k] = R(u); vy[k] = R(v); vz[k] = R(w);
+      const S w[3] = {S(f1[k]), S(f2[k]), S(f3[k])};
+      lds_corner<S, 3>(sh.rows, k, w);
     }
-    // GBUF%OFF enters the geometry; the rest of the element state is read after the
-    // kinematics (the fence keeps the compiler from hoisting the loads), so it is not
-    // live through the geometry and the kinematics
-    st.offg = e.offg[i];
-    auto load_rest = [&]() {
-      if constexpr (kStage) {
-        wait_staged();
-        const S *s = sst + threadIdx.x;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) st.sig[k] = s[k * kTile];
-        st.eint = s[6 * kTile]; st.rho = s[7 * kTile]; st.vol0 = s[8 * kTile]; st.pla = s[9 * kTile];
-        st.epsd = s[10 * kTile]; st.qvis = s[11 * kTile];
-      } else {
-        __asm__ __volatile__("" ::: "memory");
-#pragma unroll
-        for (int k = 0; k < 6; ++k) st.sig[k] = e.sig[(int64_t)k * e.ne + i];
-        st.eint = e.eint[i]; st.rho = e.rho[i]; st.vol0 = e.vol0[i]; st.pla = e.pla[i];
-        st.epsd = e.epsd[i]; st.qvis = e.qvis[i];
-      }
-    };
-    if constexpr (sizeof(R) == 8) {
-      // FP64: each node's force triple leaves for LDS as soon as it is final, which keeps
-      // the chain within two waves' register budget
-      auto write_row = [&](int k, R fx, R fy, R fz) {
-        const S w[3] = {S(fx), S(fy), S(fz)};
-        lds_corner<S, 3>(lds, k, w);
-      };
-      hex_element<R, S>(xd, yd, zd, vx, vy, vz, st, c, DT1, o, write_row, load_rest, ehou_sink);
-    } else {
-      // FP32: the forces are gathered first and stored together (registers are not the limit)
-      R f1[8], f2[8], f3[8];
-      auto keep = [&](int k, R fx, R fy, R fz) { f1[k] = fx; f2[k] = fy; f3[k] = fz; };
-      hex_element<R, S>(xd, yd, zd, vx, vy, vz, st, c, DT1, o, keep, load_rest, ehou_sink);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const S w[3] = {S(f1[k]), S(f2[k]), S(f3[k])};
-        lds_corner<S, 3>(lds, k, w);
-      }
-    }
-    if (!stopped) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) e.sig[(int64_t)k * e.ne + i] = st.sig[k];
-      e.eint[i] = st.eint; e.rho[i] = st.rho; e.pla[i] = st.pla;
-      e.epsd[i] = st.epsd; e.offg[i] = st.offg; e.qvis[i] = st.qvis;
-      if (output && M.dtel_h) to_global(M.dtel_h)[i] = o.dtx;
-    }
-    dtx = o.dtx;
-    mstop = o.mstop;
   }
   if (stopped) return; // uniform over the workgroup
-  __shared__ double red[TB / 64];
-  TileAssembly<S, kHexRowWords, 8> ta;
-  ta.prefetch(e.rest, e.ne, i, to_global(M.hfr_start), to_global(M.hfr_node), to_global<const v4u>(M.hfr_src),
-              tl.first / kTile);
-  wave_min_to(red, dtx);
-  if (mstop) atomicOr(M.flags, kMstopJacobian);
-  __syncthreads();
-  tile_min_commit<TB>(red, M.dtmin + parity);
-  if constexpr (EH) {
-    if (M.ehou_h) tile_ehou_commit<TB>(seh, tl.first, e.ne, M.ehou_h + tl.first / kTile);
+  if (active) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) e.sig[(int64_t)k * e.ne + i] = st.sig[k];
+    e.eint[i] = st.eint; e.rho[i] = st.rho; e.pla[i] = st.pla;
+    e.epsd[i] = st.epsd; e.offg[i] = st.offg; e.qvis[i] = st.qvis;
+    if (output && M.dtel_h) to_global(M.dtel_h)[i] = o.dtx;
   }
-  ta.finish(lds, to_global<S>(M.rowh), to_global(M.hfr_node), to_global<const v4u>(M.hfr_src), to_global(M.preh));
+  ta.prefetch(e.rest, e.ne, i, to_global(M.hfr_node), to_global<const v4u>(M.hfr_src));
+  wave_min_to(sh.red, active ? o.dtx : kEP06);
+  if (active && o.mstop) atomicOr(M.flags, kMstopJacobian);
+  __syncthreads();
+  tile_min_commit<kTile>(sh.red, M.dtmin + parity);
+  if constexpr (EH) {
+    if (M.ehou_h) tile_ehou_commit<kTile>(sh.seh, first, e.ne, M.ehou_h + first / kTile);
+  }
+  ta.finish(sh.rows, to_global<S>(M.rowh), to_global(M.hfr_node), to_global<const v4u>(M.hfr_src), to_global(M.preh));
+}
+
+// The tile of workgroup b of nb: the launch's tile list, or the only model's tiles in order.
+__device__ __forceinline__ Tile launch_tile(const Tile *tiles, int64_t b, int64_t nb) {
+  const int64_t t = xcd_contiguous_block(b, nb);
+  if (!tiles) return Tile{0, (int32_t)(t * kTile)};
+  const cptr<Tile> p = (cptr<Tile>)(tiles + t);
+  return Tile{p->model, p->first};
+}
+
+template <typename R, typename S, int TB, int W, bool EH>
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_hex_forces(
+    const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int parity_output) {
+  static_assert(TB == kTile, "a hex workgroup is one assembly tile");
+  __shared__ TileLds<R, S, EH, false> sh;
+  const Tile tl = launch_tile(tiles, blockIdx.x, gridDim.x);
+  hex_tile<R, S, EH>(md[tl.model], tl.first, parity_output, sh);
 }
 
 // ---------------------------------------------------------------- Q4 element kernel
+// Per-point state of a resident shell, each point loaded one point ahead, so that its loads
+// overlap the previous point's arithmetic.
 template <typename R, typename S> struct Q4IpIO {
   const Q4Ptrs<S> &q;
-  int64_t i;
-  bool active; // false: the model has stopped, nothing is stored
+  int64_t i;   // the thread's element, the last one for threads past it
+  bool active; // false: past the last element, or the model has stopped: nothing is stored
+  int npt;
+  R s_next[5], pla_next, epsd_next;
+  __device__ __forceinline__ void begin() {
+    load(0, s_next, pla_next, epsd_next);
+  }
+  __device__ __forceinline__ void fetch(int ip, R (&s)[5], R &pla, R &epsd_ip) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s[k] = s_next[k];
+    pla = pla_next; epsd_ip = epsd_next;
+    if (ip + 1 < npt) load(ip + 1, s_next, pla_next, epsd_next);
+  }
   __device__ __forceinline__ void load(int ip, R (&s)[5], R &pla, R &epsd_ip) const {
     const gptr<const S> sg = q.sig + (int64_t)ip * 5 * q.ne + i;
 #pragma unroll
@@ -534,79 +616,84 @@ template <typename R, typename S> struct Q4IpIO {
   }
 };
 
-template <typename R, typename S, int TB, int W, bool EH>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_q4_forces(
-    const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int parity_output) {
-  static_assert(TB == kTile, "a shell workgroup is one assembly tile");
-  const int parity = parity_output & 1; // bit 1: an output cycle, as for the hex kernel
+// ---------------------------------------------------------------- Q4 element tile
+// The CFORC3 chain of one tile; threads past the last element as in hex_tile.
+template <typename R, typename S, bool EH>
+__device__ __forceinline__ void q4_tile(const ModelDev &M, int64_t first, int parity_output,
+                                        TileLds<R, S, EH, sizeof(R) == 8> &sh) {
+  const int parity = parity_output & 1; // bit 1: an output cycle, as for the hex tile
   const bool output = (parity_output & 2) != 0;
-  __shared__ S lds[4 * kQ4RowWords * kTile];
-  const Tile tl = tiles[xcd_contiguous_block(blockIdx.x, gridDim.x)];
-  const ModelDev &M = md[tl.model];
   const DevTime *ts = M.ts;
   const int stopped = time_done(ts + parity); // tested before the stores only
   const Q4Ptrs<S> q = q4_ptrs<S>(M);
   const gptr<const double> xv = to_global<const double>(M.nd.xv);
   const gptr<const double> vr = to_global<const double>(M.nd.vr);
   const Q4Consts &c = M.qc;
-  const int64_t i = (int64_t)tl.first + threadIdx.x;
-  double dt = kEP06;
-  __shared__ R seh[EH ? TB : 1];
-  if (i < q.ne) {
-    const R DT1 = R(time_dt2(ts + parity));
-    double xg[4], yg[4], zg[4];
-    R vl[4][3], vrl[4][3];
-    int32_t nc[4];
+  const int64_t i = first + threadIdx.x;
+  const bool active = i < q.ne;
+  const int64_t ic = active ? i : q.ne - 1;
+  int32_t nc[4]; // node ids first, as in hex_tile
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      nc[k] = q.conn[(int64_t)k * q.ne + i];
-      double a, b, cc, u, v, w;
-      load_node(xv, nc[k], a, b, cc, u, v, w);
-      xg[k] = a; yg[k] = b; zg[k] = cc;
-      vl[k][0] = R(u); vl[k][1] = R(v); vl[k][2] = R(w);
-      const gptr<const v2d> p = (gptr<const v2d>)(vr + 4 * (int64_t)nc[k]);
-      const v2d r0 = p[0], r1 = p[1];
-      vrl[k][0] = R(r0.x); vrl[k][1] = R(r0.y); vrl[k][2] = R(r1.x);
-    }
-    Q4Elem<R> st;
-    st.offg = R(q.offg[i]); st.thk = R(q.thk[i]); st.thke = R(q.thke[i]); st.epsd = R(q.epsd[i]);
-    Q4IpIO<R, S> io{q, i, !stopped};
-    Q4Out<R> o;
-    // EH: the model keeps EHOUR (its own instantiation, so that the other keeps its registers)
-    auto ehou_sink = [&](R v) {
-      if constexpr (EH) seh[threadIdx.x] = v;
-    };
-    auto nload = [&](int k, double(&x)[3], R(&v)[3]) {
-      __asm__ __volatile__("" ::: "memory"); // a fresh load, not the values held since the gather
-      double a, b, cc, u, w, z;
-      load_node(xv, nc[k], a, b, cc, u, w, z);
-      x[0] = a; x[1] = b; x[2] = cc;
-      v[0] = R(u); v[1] = R(w); v[2] = R(z);
-    };
-    q4_element<R>(xg, yg, zg, vl, vrl, nc[2] == nc[3], st, c, DT1, io, nload, o, ehou_sink);
-    if (!stopped) {
-      q.offg[i] = S(st.offg); q.thk[i] = S(st.thk); q.epsd[i] = S(st.epsd);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const S w[6] = {S(-o.f[0][k]), S(-o.f[1][k]), S(-o.f[2][k]), S(-o.m[0][k]), S(-o.m[1][k]), S(-o.m[2][k])};
-        lds_corner<S, 6>(lds, k, w);
-      }
-      if (output && M.dtel_q) to_global(M.dtel_q)[i] = o.dt;
-    }
-    dt = o.dt;
-  }
-  if (stopped) return; // uniform over the workgroup
-  __shared__ double red[TB / 64];
+  for (int k = 0; k < 4; ++k) nc[k] = q.conn[(int64_t)k * q.ne + ic];
+  __asm__ __volatile__("" ::: "memory");
   TileAssembly<S, kQ4RowWords, 4> ta;
-  ta.prefetch(q.rest, q.ne, i, to_global(M.qfr_start), to_global(M.qfr_node), to_global<const v4u>(M.qfr_src),
-              tl.first / kTile);
-  wave_min_to(red, dt);
-  __syncthreads();
-  tile_min_commit<TB>(red, M.dtmin + parity);
-  if constexpr (EH) {
-    if (M.ehou_q) tile_ehou_commit<TB>(seh, tl.first, q.ne, M.ehou_q + tl.first / kTile);
+  ta.range(M.qfr_start, first / kTile);
+  const R DT1 = R(time_dt2(ts + parity));
+  double xg[4], yg[4], zg[4];
+  R vl[4][3], vrl[4][3];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    double a, b, cc, u, v, w;
+    load_node(xv, nc[k], a, b, cc, u, v, w);
+    xg[k] = a; yg[k] = b; zg[k] = cc;
+    vl[k][0] = R(u); vl[k][1] = R(v); vl[k][2] = R(w);
+    const gptr<const v2d> p = (gptr<const v2d>)(vr + 4 * (int64_t)nc[k]);
+    const v2d r0 = p[0], r1 = p[1];
+    vrl[k][0] = R(r0.x); vrl[k][1] = R(r0.y); vrl[k][2] = R(r1.x);
   }
-  ta.finish(lds, to_global<S>(M.rowq), to_global(M.qfr_node), to_global<const v4u>(M.qfr_src), to_global(M.preq));
+  Q4Elem<R> st;
+  st.offg = R(q.offg[ic]); st.thk = R(q.thk[ic]); st.thke = R(q.thke[ic]); st.epsd = R(q.epsd[ic]);
+  Q4IpIO<R, S> io{q, ic, active && !stopped, c.npt};
+  Q4Out<R> o;
+  // EH: the model keeps EHOUR (its own instantiation, so that the other keeps its registers)
+  auto ehou_sink = [&](R v) {
+    if constexpr (EH) sh.seh[threadIdx.x] = v;
+  };
+  auto nload = [&](int k, double(&x)[3], R(&v)[3]) {
+    __asm__ __volatile__("" ::: "memory"); // a fresh load, not the values held since the gather
+    double a, b, cc, u, w, z;
+    load_node(xv, nc[k], a, b, cc, u, w, z);
+    x[0] = a; x[1] = b; x[2] = cc;
+    v[0] = R(u); v[1] = R(w); v[2] = R(z);
+  };
+  q4_element<R>(xg, yg, zg, vl, vrl, nc[2] == nc[3], st, c, DT1, io, nload, o, ehou_sink, chain_tab<R>(sh.tab));
+  if (stopped) return; // uniform over the workgroup
+  if (active) {
+    q.offg[i] = S(st.offg); q.thk[i] = S(st.thk); q.epsd[i] = S(st.epsd);
+    if (output && M.dtel_q) to_global(M.dtel_q)[i] = o.dt;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const S w[6] = {S(-o.f[0][k]), S(-o.f[1][k]), S(-o.f[2][k]), S(-o.m[0][k]), S(-o.m[1][k]), S(-o.m[2][k])};
+    lds_corner<S, 6>(sh.rows, k, w);
+  }
+  ta.prefetch(q.rest, q.ne, i, to_global(M.qfr_node), to_global<const v4u>(M.qfr_src));
+  wave_min_to(sh.red, active ? o.dt : kEP06);
+  __syncthreads();
+  tile_min_commit<kTile>(sh.red, M.dtmin + parity);
+  if constexpr (EH) {
+    if (M.ehou_q) tile_ehou_commit<kTile>(sh.seh, first, q.ne, M.ehou_q + first / kTile);
+  }
+  ta.finish(sh.rows, to_global<S>(M.rowq), to_global(M.qfr_node), to_global<const v4u>(M.qfr_src), to_global(M.preq));
+}
+
+template <typename R, typename S, int TB, int W, bool EH>
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_q4_forces(
+    const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int parity_output) {
+  static_assert(TB == kTile, "a shell workgroup is one assembly tile");
+  __shared__ TileLds<R, S, EH, sizeof(R) == 8> sh;
+  const Tile tl = launch_tile(tiles, blockIdx.x, gridDim.x);
+  q4_tile<R, S, EH>(md[tl.model], tl.first, parity_output, sh);
 }
 
 // ---------------------------------------------------------------- nodal update pieces
@@ -663,11 +750,11 @@ __host__ __device__ __forceinline__ double dt2_pipeline(double dt2t, double dt2o
 }
 
 // ---------------------------------------------------------------- node kernel
+// Block b of a launch's list, or of the only model's nodes.
 template <typename S>
-__global__ __launch_bounds__(kBlock) void k_node_update(const ModelDev *__restrict__ md,
-                                                        const Tile *__restrict__ tiles, int parity,
-                                                        double dt_growth, int output) {
-  const Tile tl = tiles[blockIdx.x];
+__device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int32_t b,
+                                          int parity, double dt_growth, int output) {
+  const Tile tl = tiles ? tiles[b] : Tile{0, b * kBlock};
   const ModelDev &M = md[tl.model];
   const NodePtrs &nd = M.nd;
   const gptr<const S> rowh = to_global<const S>(M.rowh);
@@ -835,6 +922,13 @@ __global__ __launch_bounds__(kBlock) void k_node_update(const ModelDev *__restri
   p[0] = v2d{x, y};
   p[1] = v2d{z, vx};
   p[2] = v2d{vy, vz};
+}
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_node_update(const ModelDev *__restrict__ md,
+                                                        const Tile *__restrict__ tiles, int parity,
+                                                        double dt_growth, int output) {
+  node_tile<S>(md, tiles, (int32_t)blockIdx.x, parity, dt_growth, output);
 }
 
 // ---------------------------------------------------------------- energies (fixed-order)
@@ -1028,6 +1122,15 @@ __global__ __launch_bounds__(kBlock) void k_sforc3_group(int nel, int64_t nft, c
 struct GroupIpIO {
   double *sig, *pla, *epsd_ip, *gstr, *hourg, *eint, *forc, *mom;
   int nel, i;
+  double s_next[5], pla_next, epsd_next; // each point's state, loaded one point ahead
+  int npt;
+  __device__ __forceinline__ void begin() { load(0, s_next, pla_next, epsd_next); }
+  __device__ __forceinline__ void fetch(int ip, double (&s)[5], double &p, double &e) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s[k] = s_next[k];
+    p = pla_next; e = epsd_next;
+    if (ip + 1 < npt) load(ip + 1, s_next, pla_next, epsd_next);
+  }
   __device__ __forceinline__ void late_load(Q4Late<double> &L) const {
 #pragma unroll
     for (int k = 0; k < 5; ++k) L.forc[k] = forc[(int64_t)k * nel + i];
@@ -1093,6 +1196,7 @@ __global__ __launch_bounds__(kBlock) void k_cforc3_group(int nel, int64_t nft, c
   Q4Elem<double> st;
   st.offg = offg[i]; st.thk = thk[i]; st.thke = thke[i]; st.epsd = epsd[i];
   GroupIpIO io{sig, pla, epsd_ip, gstr, hourg, eint, forc, mom, nel, i};
+  io.npt = c.npt;
   Q4Out<double> o;
   auto nload = [&](int k, double(&p)[3], double(&w)[3]) {
     const int64_t n = (int64_t)nc[k] - 1;
@@ -1323,13 +1427,12 @@ struct or_model {
   int32_t *lidx_h = nullptr, *lidx_q = nullptr;
   unsigned long long *ctrl = nullptr;  // [4]
   int64_t parity = 0;
-  // what the kernels see (host copy, device copy) and the model's own tile lists
+  // what the kernels see (host copy, device copy) and the numbers of its tiles
   ModelDev hdev{};
   ModelDev *dev = nullptr;
   bool dev_dirty = true;
-  Tile *tiles_h = nullptr, *tiles_q = nullptr, *tiles_n = nullptr;
   int32_t nt_h = 0, nt_q = 0, nt_n = 0;
-  int var_h = 0, var_q = 0;            // element kernel variants (tiles_h / tiles_q follow their block)
+  int var_h = 0, var_q = 0;            // element kernel variants
   or_batch *batch = nullptr;           // set while the model belongs to a batch
   // timing
   bool timing = false;
@@ -1374,19 +1477,6 @@ static void mark_changed(or_model *m) {
 }
 
 static size_t ssize(const or_model *m) { return m->prec == OR_PREC_FP64 ? sizeof(double) : sizeof(float); }
-
-// Element tiles of a model alone, for its current variants.
-static int put_elem_tiles(or_model *m) {
-  for (int f = 0; f < 2; ++f) {
-    const int64_t ne = f == 0 ? m->neh : m->neq;
-    if (ne == 0) continue;
-    std::vector<Tile> tl;
-    for (int64_t first = 0; first < ne; first += kTile) tl.push_back(Tile{0, (int32_t)first});
-    OR_HIP(hipMemcpy(f == 0 ? m->tiles_h : m->tiles_q, tl.data(), sizeof(Tile) * tl.size(), hipMemcpyHostToDevice));
-    (f == 0 ? m->nt_h : m->nt_q) = (int32_t)tl.size();
-  }
-  return OR_OK;
-}
 
 // Entry points: C linkage comes from their declarations in or_gpu.h.
 
@@ -1484,9 +1574,8 @@ int or_model_create(or_model **out, int device, int64_t nn, int64_t ne_hex, int6
   A(&m->flags, 1);
   A(&m->dev, 1);
   m->nt_n = (int32_t)((nn + kBlock - 1) / kBlock);
-  A(&m->tiles_h, (ne_hex + kTile - 1) / kTile);
-  A(&m->tiles_q, (ne_q4 + kTile - 1) / kTile);
-  A(&m->tiles_n, m->nt_n);
+  m->nt_h = (int32_t)((ne_hex + kTile - 1) / kTile);
+  m->nt_q = (int32_t)((ne_q4 + kTile - 1) / kTile);
   const int64_t nb = 1024;
   A(&m->energy, kEnergySums * (1 + nb));
   if (rc == OR_OK && hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess)
@@ -1505,16 +1594,6 @@ int or_model_create(or_model **out, int device, int64_t nn, int64_t ne_hex, int6
     double big = kEP06;
     std::memcpy(&dm[0], &big, 8);
     dm[1] = dm[0];
-    std::vector<Tile> tl;
-    auto put_tiles = [&](Tile *dst, int32_t nt) {
-      if (rc != OR_OK || nt == 0) return;
-      tl.resize((size_t)nt);
-      for (int32_t b = 0; b < nt; ++b) tl[(size_t)b] = Tile{0, b * kBlock};
-      if (hipMemcpy(dst, tl.data(), sizeof(Tile) * (size_t)nt, hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(OR_ERR_HIP, "tile upload");
-    };
-    put_tiles(m->tiles_n, m->nt_n);
-    if (rc == OR_OK) rc = put_elem_tiles(m);
     if (rc == OR_OK && (hipMemcpyAsync(m->ts, tsh, sizeof(tsh), hipMemcpyHostToDevice, m->stream) != hipSuccess ||
                         hipMemcpyAsync(m->dtmin, dm, sizeof(dm), hipMemcpyHostToDevice, m->stream) != hipSuccess ||
                         hipStreamSynchronize(m->stream) != hipSuccess))
@@ -1541,7 +1620,7 @@ int or_model_destroy(or_model *m) {
                   m->qrest, m->qfr_start, m->qfr_node, m->qfr_src, m->qoffg, m->qthk, m->qthke, m->qforc, m->qmom,
                   m->qgstr, m->qhourg, m->qeint, m->qepsd,
                   m->qsig, m->qpla, m->qepsdip, m->rowq, m->ts, m->dtmin, m->flags, m->energy, m->dev,
-                  m->tiles_h, m->tiles_q, m->tiles_n, m->ecrit, m->wext, m->dtel_h, m->dtel_q, m->lidx_h,
+                  m->ecrit, m->wext, m->dtel_h, m->dtel_q, m->lidx_h,
                   m->lidx_q, m->ctrl, m->th_slot, m->th_hex, m->th_q4, m->th_buf, m->ehou_h, m->ehou_q};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -1973,8 +2052,8 @@ static int refresh_dev(or_model *m) {
 
 #endif // OR_ILP_TU
 
-// The three launches of one cycle for a set of models of one precision: element
-// forces (hexes, then shells) and the node update, each over the set's tile list.
+// The launches of one cycle for a set of models of one precision: element forces (hexes and
+// shells) and the node update, each over the set's tile list (null: one model's own tiles).
 struct LaunchSet {
   const ModelDev *md = nullptr;
   const Tile *th = nullptr, *tq = nullptr, *tn = nullptr;
@@ -2033,6 +2112,16 @@ void or_ilp_elements(int family, int fp64, int variant, hipStream_t st, const vo
 #else
 ;
 
+static LaunchSet model_set(const or_model *m) {
+  LaunchSet L;
+  L.md = m->dev;
+  L.nth = m->nt_h; L.vh = m->var_h;
+  L.eh = m->ehou_h != nullptr; L.eq = m->ehou_q != nullptr;
+  L.ntq = m->nt_q; L.vq = m->var_q;
+  L.ntn = m->nt_n;
+  return L;
+}
+
 template <typename R, typename S>
 static int launch_cycle(hipStream_t st, const LaunchSet &L, int parity, hipEvent_t after_hex, hipEvent_t after_q4,
                         int output = 0) {
@@ -2068,12 +2157,7 @@ int or_model_run(or_model *m, int64_t ncycles) {
   OR_HIP(hipSetDevice(m->device));
   int rc0 = refresh_dev(m);
   if (rc0) return rc0;
-  LaunchSet L;
-  L.md = m->dev;
-  L.th = m->tiles_h; L.nth = m->nt_h; L.vh = m->var_h;
-  L.eh = m->ehou_h != nullptr; L.eq = m->ehou_q != nullptr;
-  L.tq = m->tiles_q; L.ntq = m->nt_q; L.vq = m->var_q;
-  L.tn = m->tiles_n; L.ntn = m->nt_n;
+  const LaunchSet L = model_set(m);
   for (int64_t c = 0; c < ncycles; ++c) {
     if (m->timing) {
       if (m->ring_used * 4 + 4 > (int)m->ev.size()) {
@@ -2149,12 +2233,7 @@ int or_model_run_ecrit(or_model *m, or_ecrit *out) {
   if ((rc = fill_ep06(m->dtel_h, m->neh)) || (rc = fill_ep06(m->dtel_q, m->neq))) return rc;
   rc = refresh_dev(m);
   if (rc) return rc;
-  LaunchSet L;
-  L.md = m->dev;
-  L.th = m->tiles_h; L.nth = m->nt_h; L.vh = m->var_h;
-  L.eh = m->ehou_h != nullptr; L.eq = m->ehou_q != nullptr;
-  L.tq = m->tiles_q; L.ntq = m->nt_q; L.vq = m->var_q;
-  L.tn = m->tiles_n; L.ntn = m->nt_n;
+  const LaunchSet L = model_set(m);
   const int p = (int)(m->parity & 1);
   rc = (m->prec == OR_PREC_FP64) ? launch_cycle<double, double>(m->stream, L, p, nullptr, nullptr, 1)
                                  : launch_cycle<float, float>(m->stream, L, p, nullptr, nullptr, 1);
@@ -2492,7 +2571,6 @@ int or_model_footprint_estimate(int64_t nn, int64_t ne_hex, int64_t ne_q4, int32
   if (precision != OR_PREC_FP64 && precision != OR_PREC_SPLIT) return fail(OR_ERR_ARG, "bad precision");
   if ((ne_hex > 0 && !rows_hex) || (ne_q4 > 0 && !rows_q4)) return fail(OR_ERR_ARG, "missing row counts");
   const int64_t ss = precision == OR_PREC_FP64 ? 8 : 4;
-  const int64_t nsl = (nn + kBlock - 1) / kBlock;
   const int64_t th = (ne_hex + kTile - 1) / kTile, tq = (ne_q4 + kTile - 1) / kTile;
   // the allocations of or_model_create, in the same order
   int64_t b = 8 * (6 * nn + 3 * nn + nn + 3 * nn) + 4 * nn;             // xv, d, ms, vimp, code
@@ -2506,7 +2584,6 @@ int or_model_footprint_estimate(int64_t nn, int64_t ne_hex, int64_t ne_q4, int32
     if (strain_rate_filter) b += ss * (int64_t)npt * ne_q4;              // LBUF EPSD (or_model_set_q4_params)
   }
   b += (int64_t)sizeof(DevTime) * 2 + 8 * 2 + 4 + 8 * (kEnergySums * (1 + 1024)) + (int64_t)sizeof(ModelDev);
-  b += (int64_t)sizeof(Tile) * (th + tq + nsl);
   // or_model_upload_skyline: rest rows (at most every row of the family) and the prefix lists
   // (at most one prefix per node and family)
   for (int f = 0; f < 2; ++f) {
@@ -3030,7 +3107,7 @@ int or_model_set_variant(or_model *m, int family, int variant) {
   OR_HIP(hipSetDevice(m->device));
   OR_HIP(quiesce(m));
   (family == 0 ? m->var_h : m->var_q) = variant;
-  return put_elem_tiles(m);
+  return OR_OK;
 }
 
 int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]) {
@@ -3049,12 +3126,7 @@ int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]
     float best_ms = 0.f;
     for (int v = 0; v < kVariants; ++v) {
       if ((rc = or_model_set_variant(m, f, v))) return rc;
-      LaunchSet L;
-      L.md = m->dev;
-      L.th = m->tiles_h; L.nth = m->nt_h; L.vh = m->var_h;
-      L.eh = m->ehou_h != nullptr; L.eq = m->ehou_q != nullptr;
-      L.tq = m->tiles_q; L.ntq = m->nt_q; L.vq = m->var_q;
-      L.tn = m->tiles_n; L.ntn = m->nt_n;
+      const LaunchSet L = model_set(m);
       float ms = 0.f;
       auto one = [&]() -> int {
         const int p = (int)(m->parity & 1);

@@ -41,20 +41,21 @@ template <typename T> __device__ __forceinline__ T dminT(T a, T b) { return (a <
 
 // FP64: the correctly rounded double-double routines of or_math.h; FP32 (split
 // form): the device library.
-__device__ __forceinline__ double powR(double a, double b) { return ormath::or_pow(a, b); }
-__device__ __forceinline__ float powR(float a, float b) { return powf(a, b); }
+template <class T> __device__ __forceinline__ double powR(double a, double b, T tab) { return ormath::or_pow(a, b, tab); }
+template <class T> __device__ __forceinline__ float powR(float a, float b, T) { return powf(a, b); }
 // a**b1 and a**b2 (FP64: one shared logarithm, the results of two powR calls)
-__device__ __forceinline__ void pow2R(double a, double b1, double b2, double &r1, double &r2) {
-  ormath::or_pow2(a, b1, b2, r1, r2);
+template <class T>
+__device__ __forceinline__ void pow2R(double a, double b1, double b2, double &r1, double &r2, T tab) {
+  ormath::or_pow2(a, b1, b2, r1, r2, tab);
 }
-__device__ __forceinline__ void pow2R(float a, float b1, float b2, float &r1, float &r2) {
+template <class T> __device__ __forceinline__ void pow2R(float a, float b1, float b2, float &r1, float &r2, T) {
   r1 = powf(a, b1);
   r2 = powf(a, b2);
 }
 __device__ __forceinline__ double sqrtR(double a) { return sqrt(a); }
 __device__ __forceinline__ float sqrtR(float a) { return sqrtf(a); }
-__device__ __forceinline__ double logR(double a) { return ormath::or_log(a); }
-__device__ __forceinline__ float logR(float a) { return logf(a); }
+template <class T> __device__ __forceinline__ double logR(double a, T tab) { return ormath::or_log(a, tab); }
+template <class T> __device__ __forceinline__ float logR(float a, T) { return logf(a); }
 __device__ __forceinline__ double fabsR(double a) { return fabs(a); }
 __device__ __forceinline__ float fabsR(float a) { return fabsf(a); }
 
@@ -308,10 +309,10 @@ __device__ __forceinline__ void hex_kinematics(R (&vx)[8], R (&vy)[8], R (&vz)[8
 
 // Material and forces: SRHO3, SROTA3, MMAIN / M2LAW, MSTRAIN_RATE, MQVISCB, SMALLB3,
 // SHVIS3 forces, SFINT3, SCUMU3P.  Updates the element state st and fills o.
-template <typename R, typename S, typename Write, typename Ehou = NoEhou>
+template <typename R, typename S, typename Write, typename Ehou = NoEhou, class T = ormath::GlobalTab>
 __device__ __forceinline__ void hex_material_forces(const HexGeom<R> &g, const HexKin<R> &kn, HexState<S> &st,
                                                     const HexConsts &c, const R DT1, HexOut<R> &o, Write &&write,
-                                                    Ehou ehou_sink = Ehou{}) {
+                                                    Ehou ehou_sink = Ehou{}, const T tab = T{}) {
   const R ZERO = R(0), ONE = R(1), TWO = R(2), THREE = R(3);
   const R HALF = R(1.0 / 2.0), THIRD = R(1.0 / 3.0), FOURTH = R(1.0 / 4.0);
   const R TWO_THIRD = R(2.0 / 3.0), HUNDRED = R(100.0);
@@ -395,10 +396,10 @@ __device__ __forceinline__ void hex_material_forces(const HexGeom<R> &g, const H
   if (c.cc != 0.0) {
     if (c.vp == 1) {
       EPD = dmaxT(epsd, R(c.epdr));
-      EPD = logR(EPD / R(c.epdr));
+      EPD = logR(EPD / R(c.epdr), tab);
     } else {
       EPD = dmaxT(epsd, EM15);
-      EPD = logR(EPD / R(c.epdr));
+      EPD = logR(EPD / R(c.epdr), tab);
     }
     EPD = dmaxT(ZERO, EPD);
     EPD = (ONE + R(c.cc) * EPD) * ONE;
@@ -412,7 +413,7 @@ __device__ __forceinline__ void hex_material_forces(const HexGeom<R> &g, const H
     QH = CB * EPD;
   } else if (epxe > ZERO) {
     R pn, pq; // EPXE**CN, and EPXE**(CN-1) or EPXE**(1-CN)
-    pow2R(epxe, CN, (CN > ONE) ? CN - ONE : ONE - CN, pn, pq);
+    pow2R(epxe, CN, (CN > ONE) ? CN - ONE : ONE - CN, pn, pq, tab);
     AK = R(c.ca) + CB * pn;
     if (CN > ONE) QH = (CB * CN * pq) * EPD;
     else QH = (CB * CN / pq) * EPD;
@@ -440,8 +441,8 @@ __device__ __forceinline__ void hex_material_forces(const HexGeom<R> &g, const H
     R AD = ZERO, AL = ZERO;
     R CX = SSP + ZERO; // SSP + SQRT(VD2), VD2 = 0
     // AL = VOLN**(1/3) here and VOLN**(2/3) of SHVIS3 below, from one logarithm of VOLN
-    if (off == ONE && VOLN > ZERO) pow2R(VOLN, ONE / THREE, TWO_THIRD, AL, vol23);
-    else vol23 = powR(VOLN, TWO_THIRD);
+    if (off == ONE && VOLN > ZERO) pow2R(VOLN, ONE / THREE, TWO_THIRD, AL, vol23, tab);
+    else vol23 = powR(VOLN, TWO_THIRD, tab);
     if (off == ONE) AD = dmaxT(ZERO, DD);
     R NRHO = sqrtR(rhoref * RHO0);
     R QA = ONE * R(c.qa), QB = ONE * R(c.qb);
@@ -583,17 +584,18 @@ __device__ __forceinline__ void hex_material_forces(const HexGeom<R> &g, const H
 
 // The whole chain for one element.  st.offg and the gathered nodes are read beforehand;
 // load_rest() reads the rest of st between the kinematics and the material phase.
-template <typename R, typename S, typename Write, typename LoadRest, typename Ehou = NoEhou>
+template <typename R, typename S, typename Write, typename LoadRest, typename Ehou = NoEhou,
+          class T = ormath::GlobalTab>
 __device__ __forceinline__ void hex_element(const double (&xd)[8], const double (&yd)[8], const double (&zd)[8],
                                             R (&vx)[8], R (&vy)[8], R (&vz)[8], HexState<S> &st,
                                             const HexConsts &c, const R DT1, HexOut<R> &o, Write &&write,
-                                            LoadRest &&load_rest, Ehou ehou_sink = Ehou{}) {
+                                            LoadRest &&load_rest, Ehou ehou_sink = Ehou{}, const T tab = T{}) {
   HexGeom<R> g;
   hex_geometry<R>(xd, yd, zd, double(st.offg), g);
   HexKin<R> kn;
   hex_kinematics<R>(vx, vy, vz, g, DT1, kn);
   load_rest();
-  hex_material_forces<R, S>(g, kn, st, c, DT1, o, write, ehou_sink);
+  hex_material_forces<R, S>(g, kn, st, c, DT1, o, write, ehou_sink, tab);
 }
 
 } // namespace orgpu

@@ -50,16 +50,16 @@ template <typename R> struct Q4Out {
   R ehou;       // CHVIS3's hourglass energy of the cycle (EHOU)
 };
 
-__device__ __forceinline__ double expR(double a) { return ormath::or_exp(a); }
-__device__ __forceinline__ float expR(float a) { return expf(a); }
+template <class T> __device__ __forceinline__ double expR(double a, T tab) { return ormath::or_exp(a, tab); }
+template <class T> __device__ __forceinline__ float expR(float a, T) { return expf(a); }
 template <typename T> __device__ __forceinline__ T fsignT(T a, T b) { return copysign(fabs(a), b); }
 
 // M2CPLR (m2cplr.F) for one integration point, IFORM=0, FISOKIN=0, IMPL_S=0.
 // off is OFF_OLD, the element OFF before this cycle's rupture test (sigeps02c.F:135).
-template <typename R>
+template <typename R, class T>
 __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, const R a2, const R epdr, R off, R gs,
                                              R epsp_in, R (&s)[5], R dxx, R dyy, R dxy, R dyz, R dzx, R &pla,
-                                             R &ezz, R &epchk) {
+                                             R &ezz, R &epchk, T &tab) {
   const R ZERO = R(0), ONE = R(1), TWO = R(2), THREE = R(3), HALF = R(0.5), FOURTH = R(0.25);
   const R EM20 = R(1.0 / 1.0e20), EM15 = R(1.0 / 1.0e15), SMALL = R(1.0 / 1.0e7);
   const R YOUNG = R(c.young), G = R(c.shear), CN = R(c.cn);
@@ -70,11 +70,12 @@ __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, cons
   R sxy = s[2] + G * dxy;
   R syz = s[3] + gs * dyz;
   R szx = s[4] + gs * dzx;
+  tab.need(pla != ZERO || c.cc != 0.0);
   if (c.cc != 0.0) {
     R epsp = epsp_in;
     if (c.israte == 0 && c.vp == 2) epsp = dmaxT(dmaxT(fabsR(dxx), fabsR(dyy)), HALF * fabsR(dxy));
     epsp = dmaxT(epsp, epdr);
-    R logep = logR(epsp / epdr);
+    R logep = logR(epsp / epdr, tab);
     R q = (ONE + R(c.cc) * logep);
     q = dmaxT(q, EM20);
     CA = CA * q;
@@ -83,7 +84,7 @@ __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, cons
   }
   R YLD;
   if (pla == ZERO) YLD = CA;
-  else YLD = CA + (CB * (ONE - ZERO)) * expR(CN * logR(pla));
+  else YLD = CA + (CB * (ONE - ZERO)) * expR(CN * logR(pla, tab), tab);
   YLD = dminT(YLD, YMAX);
   if (c.ipla == 0) {
     R svm = sqrtR(sxx * sxx + syy * syy - sxx * syy + THREE * sxy * sxy);
@@ -101,11 +102,12 @@ __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, cons
     R A = FOURTH * s1 * s1;
     R B = R(3.0 / 4.0) * s2 * s2 + THREE * s3 * s3;
     R svm = sqrtR(A + B);
+    tab.need(svm > YLD && off == ONE);
     if (svm > YLD && off == ONE) {
       const R nu = R(c.nu);
       R nu1 = ONE / (ONE - nu), nu2 = ONE / (ONE + nu);
       if (YLD >= YMAX) H = ZERO;
-      else H = CN * CB * expR((CN - ONE) * logR(pla + SMALL));
+      else H = CN * CB * expR((CN - ONE) * logR(pla + SMALL, tab), tab);
       R dpla_j = (svm - YLD) / (THREE * G + H);
       R anu1 = A * nu1, bnu2 = THREE * B * nu2, h2 = TWO * H;
       R dpla_i = ZERO, P = ONE, Q = ONE, DR = ZERO;
@@ -115,7 +117,7 @@ __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, cons
         R pla_i = pla + dpla_i;
         R yld_i;
         if (pla_i == ZERO) yld_i = dminT(YMAX, CA);
-        else yld_i = dminT(YMAX, CA + CB * expR(CN * logR(pla_i)));
+        else yld_i = dminT(YMAX, CA + CB * expR(CN * logR(pla_i, tab), tab));
         DR = HALF * YOUNG * dpla_i / yld_i;
         P = ONE / (ONE + DR * nu1);
         Q = ONE / (ONE + THREE * DR * nu2);
@@ -138,9 +140,10 @@ __device__ __forceinline__ void m2cplr_point(const Q4Consts &c, const R a1, cons
     R svm2 = sxx * sxx + syy * syy - sxx * syy + THREE * sxy * sxy;
     R svm = sqrtR(svm2);
     R yld2 = YLD * YLD;
+    tab.need(svm2 > yld2 && off == ONE);
     if (svm2 > yld2 && off == ONE) {
       if (YLD >= YMAX) H = ZERO;
-      else H = CN * CB * expR((CN - ONE) * logR(pla + SMALL));
+      else H = CN * CB * expR((CN - ONE) * logR(pla + SMALL, tab), tab);
       R aa = (svm2 - yld2) / (R(5) * svm2 + THREE * (-sxx * syy + sxy * sxy));
       R s1 = (ONE - TWO * aa) * sxx + aa * syy;
       R s2 = aa * sxx + (ONE - TWO * aa) * syy;
@@ -211,17 +214,17 @@ __device__ __forceinline__ void q4_frame(const double (&xg)[4], const double (&y
 
 // The CFORC3 chain for one element.  xg/yg/zg: gathered coordinates (FP64);
 // vl/vrl: gathered velocities and rotational velocities; tri: node 3 == node 4.
-// sig/pla/epsd_ip: per-point state, loaded and stored by the caller through the
-// accessor ip_io (so that the kernel chooses the memory layout), which also reads
+// sig/pla/epsd_ip: per-point state, read (begin before the loop, fetch at each point) and stored by
+// the caller through the accessor ip_io (so that the kernel chooses the memory layout), which also reads
 // and writes FOR, MOM, STRA, HOURG and EINT (Q4Late).  nload(k, x, v) gives node k's coordinates and
 // velocity again after the through-thickness loop (the values of xg/yg/zg and vl), from
 // which the frame and the local velocities that CHVIS3 and CFINT3 use are formed again
 // rather than kept live across the loop.
-template <typename R, typename IPIO, typename NLOAD, typename Ehou = NoEhou>
+template <typename R, typename IPIO, typename NLOAD, typename Ehou = NoEhou, class T = ormath::GlobalTab>
 __device__ __forceinline__ void q4_element(const double (&xg)[4], const double (&yg)[4], const double (&zg)[4],
                                            R (&vl)[4][3], R (&vrl)[4][3], bool tri, Q4Elem<R> &st,
                                            const Q4Consts &c, const R DT1, IPIO &ip_io, NLOAD &&nload,
-                                           Q4Out<R> &o, Ehou ehou_sink = Ehou{}) {
+                                           Q4Out<R> &o, Ehou ehou_sink = Ehou{}, T tab = T{}) {
   const R ZERO = R(0), ONE = R(1), TWO = R(2), THREE = R(3), HALF = R(0.5), FOURTH = R(0.25);
   const R EM20 = R(1.0 / 1.0e20), EM01 = R(1.0 / 10.0);
   const R FOUR_OVER_5 = R(4.0 / 5.0);
@@ -358,23 +361,19 @@ __device__ __forceinline__ void q4_element(const double (&xg)[4], const double (
   const R epdr = dmaxT(R(c.epdr) * DT1, EM20);
   const R asrate = (c.israte > 0) ? dminT(ONE, R(c.asrate) * DT1) : ONE;
   const R nu = R(c.nu);
-  // each point's state is loaded one point ahead, so that its loads overlap the
-  // previous point's arithmetic
-  R s_next[5], pla_next, epsd_next;
-  ip_io.load(0, s_next, pla_next, epsd_next);
+  ip_io.begin();
   for (int ip = 0; ip < c.npt; ++ip) {
     const R thkly = R(c.wf[ip]);
     const R wmc = R(c.wm[ip]);
     const R thklyl = thkly * thk0;
     const R zt = (R(c.z0[ip]) + ZERO) * thk0;
     const R dxx = EXX + zt * KXX, dyy = EYY + zt * KYY, dxy = EXY + zt * KXY;
-    R s[5] = {s_next[0], s_next[1], s_next[2], s_next[3], s_next[4]};
-    R pla = pla_next, epsd_ip = epsd_next;
-    if (ip + 1 < c.npt) ip_io.load(ip + 1, s_next, pla_next, epsd_next);
+    R s[5], pla, epsd_ip;
+    ip_io.fetch(ip, s, pla, epsd_ip);
     epsd_ip = asrate * epsd_pg + (ONE - asrate) * epsd_ip;
     const R epsdot = epsd_ip * DT1;
     R ezz;
-    m2cplr_point<R>(c, a1, a2, epdr, off_old, GS, epsdot, s, dxx, dyy, dxy, EYZ, EXZ, pla, ezz, epchk);
+    m2cplr_point<R>(c, a1, a2, epdr, off_old, GS, epsdot, s, dxx, dyy, dxy, EYZ, EXZ, pla, ezz, epchk, tab);
     if (off == off_old && off > ZERO) {
       if (off == ONE && epchk >= R(c.epmx)) {
         off = FOUR_OVER_5;

@@ -51,3 +51,15 @@ def test_special_arguments(gpu_lib):
     assert np.array_equal(E.math_eval("exp", z), host("exp", z))
     w = np.array([1.0, 2.0, 1e-300, 1e300, 0.75, 1.5 - 2.0 ** -52])
     assert np.array_equal(E.math_eval("log", w), host("log", w))
+
+
+@pytest.mark.parametrize("fn", ["log", "exp", "pow"])
+def test_arguments_the_rounding_test_rejects(fn, gpu_lib):
+    """The device's short evaluation accepts a value only when its error cannot change the rounding;
+    near 1 (log) and for tiny exponents (exp, pow) nearly every argument is rejected and takes the
+    double-double path: both sides of the test give the host's bits."""
+    print(f"case: or_math_eval {fn}, arguments next to 1 and 0", flush=True)
+    t = np.ldexp(np.random.default_rng(5).uniform(1.0, 2.0, 60_000), -np.repeat(np.arange(1, 61), 1000))
+    t = np.concatenate([t, -t])
+    x, y = {"log": (1.0 + 0.5 * t, None), "exp": (t, None), "pow": (1.0 + 0.5 * t, 1.0 / 3.0)}[fn]
+    assert np.array_equal(E.math_eval(fn, x, y), host(fn, x, y))
