@@ -54,9 +54,9 @@ constexpr int kBlock = 256;
 constexpr double kNoEnd = 1.0e300; // end time of a model advanced by or_model_run
 
 // Launch variants of the element kernels.  Variant v picks the minimum number of waves
-// per SIMD the register allocation is built for (two for even v, three for odd v, where
-// the FP64 kernels spill to scratch; a wave's register budget is 512 / waves VGPRs and
-// AGPRs together) and the instruction scheduler (default for v < 2, ILP-first for v >= 2).
+// per SIMD the register allocation is built for (split form: two for even v, three for odd
+// v; FP64: two, since three spill to scratch; a wave's register budget is 512 / waves VGPRs
+// and AGPRs together) and the instruction scheduler (default for v < 2, ILP-first for v >= 2).
 // Every element workgroup is one tile of kTile elements, the unit of the LDS assembly.
 // Every variant runs the same arithmetic, so the choice (or_model_set_variant,
 // or_model_autotune, or_batch_autotune) changes speed only, never a result bit.
@@ -696,6 +696,54 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W))) void k_
   q4_tile<R, S, EH>(md[tl.model], tl.first, parity_output, sh);
 }
 
+// ---------------------------------------------------------------- all families in one launch
+// The element tiles of a cycle whose model (or batch) has more than one family or form, in one
+// launch: family f's list is t[f] (null: the only model's tiles in order) of n[f] tiles.
+// Shells come first, their chains being the longer ones.  MASK: the families compiled in.
+enum { kFamQ4 = 0, kFamHex = 1, kFamQ4Split = 2, kFamHexSplit = 3 };
+struct ElemLists {
+  const Tile *t[4];
+  int32_t n[4];
+};
+template <int MASK, bool EH>
+__global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(2))) void k_elements(
+    const ModelDev *__restrict__ md, ElemLists L, int parity_output) {
+  typedef TileLds<double, double, EH, true> Lds64;
+  typedef TileLds<double, double, EH, false> LdsHex64;
+  typedef TileLds<float, float, EH, false> Lds32;
+  __shared__ __align__(16) unsigned char buf[(MASK & 3) ? sizeof(Lds64) : sizeof(Lds32)];
+  static_assert(sizeof(Lds32) <= sizeof(Lds64), "the FP64 layout is the larger one");
+  int32_t b = (int32_t)blockIdx.x;
+  if constexpr (MASK & (1 << kFamQ4)) {
+    if (b < L.n[kFamQ4]) {
+      const Tile tl = launch_tile(L.t[kFamQ4], b, L.n[kFamQ4]);
+      q4_tile<double, double, EH>(md[tl.model], tl.first, parity_output, *(Lds64 *)buf);
+      return;
+    }
+    b -= L.n[kFamQ4];
+  }
+  if constexpr (MASK & (1 << kFamQ4Split)) {
+    if (b < L.n[kFamQ4Split]) {
+      const Tile tl = launch_tile(L.t[kFamQ4Split], b, L.n[kFamQ4Split]);
+      q4_tile<float, float, EH>(md[tl.model], tl.first, parity_output, *(Lds32 *)buf);
+      return;
+    }
+    b -= L.n[kFamQ4Split];
+  }
+  if constexpr (MASK & (1 << kFamHex)) {
+    if (b < L.n[kFamHex]) {
+      const Tile tl = launch_tile(L.t[kFamHex], b, L.n[kFamHex]);
+      hex_tile<double, double, EH>(md[tl.model], tl.first, parity_output, *(LdsHex64 *)buf);
+      return;
+    }
+    b -= L.n[kFamHex];
+  }
+  if constexpr (MASK & (1 << kFamHexSplit)) {
+    const Tile tl = launch_tile(L.t[kFamHexSplit], b, L.n[kFamHexSplit]);
+    hex_tile<float, float, EH>(md[tl.model], tl.first, parity_output, *(Lds32 *)buf);
+  }
+}
+
 // ---------------------------------------------------------------- nodal update pieces
 // ACCELE (accele.F:65-80, 97-109): A = F / MS, zero where the mass (inertia) is not positive.
 __device__ __forceinline__ void accele3(double &a0, double &a1, double &a2, double mass) {
@@ -929,6 +977,17 @@ __global__ __launch_bounds__(kBlock) void k_node_update(const ModelDev *__restri
                                                         const Tile *__restrict__ tiles, int parity,
                                                         double dt_growth, int output) {
   node_tile<S>(md, tiles, (int32_t)blockIdx.x, parity, dt_growth, output);
+}
+
+// The node update of a batch with members of both forms, in one launch: n64 blocks of FP64
+// members, then those of the split form.
+__global__ __launch_bounds__(kBlock) void k_node_update_both(const ModelDev *__restrict__ md,
+                                                             const Tile *__restrict__ t64, int32_t n64,
+                                                             const Tile *__restrict__ t32, int parity,
+                                                             double dt_growth) {
+  const int32_t b = (int32_t)blockIdx.x;
+  if (b < n64) node_tile<double>(md, t64, b, parity, dt_growth, 0);
+  else node_tile<float>(md, t32, b - n64, parity, dt_growth, 0);
 }
 
 // ---------------------------------------------------------------- energies (fixed-order)
@@ -2122,11 +2181,33 @@ static LaunchSet model_set(const or_model *m) {
   return L;
 }
 
+// A set's element kernels run in one launch (k_elements) when both families are there, their
+// variants are the default one and nobody asked for the families' own times: the tiles of one
+// family fill the compute units that the other leaves idle.  Against one launch each: 13,824
+// hexes + 2,304 shells 20.7 us a cycle (29.8), 512,000 + 160,000 141.0 (151.2; split form 93.9 and
+// 104.4), a batch of 12 bars and tubes in both forms 47.0 (103.2).
+static bool one_launch(const LaunchSet &L) { return L.nth > 0 && L.ntq > 0 && L.vh == 0 && L.vq == 0; }
+
 template <typename R, typename S>
 static int launch_cycle(hipStream_t st, const LaunchSet &L, int parity, hipEvent_t after_hex, hipEvent_t after_q4,
                         int output = 0) {
   constexpr int fp64 = sizeof(R) == 8 ? 1 : 0;
   const int po = parity | (output ? 2 : 0); // element kernels: parity and the output-cycle bit
+  if (one_launch(L) && !after_hex && !after_q4) {
+    constexpr int q = fp64 ? kFamQ4 : kFamQ4Split, h = fp64 ? kFamHex : kFamHexSplit;
+    constexpr int mask = (1 << q) | (1 << h);
+    ElemLists E{};
+    E.t[q] = L.tq; E.n[q] = L.ntq;
+    E.t[h] = L.th; E.n[h] = L.nth;
+    const dim3 g((unsigned)(L.ntq + L.nth));
+    if (L.eh || L.eq) hipLaunchKernelGGL((k_elements<mask, true>), g, dim3(kTile), 0, st, L.md, E, po);
+    else hipLaunchKernelGGL((k_elements<mask, false>), g, dim3(kTile), 0, st, L.md, E, po);
+    OR_HIP(hipGetLastError());
+    hipLaunchKernelGGL((k_node_update<S>), dim3((unsigned)L.ntn), dim3(kBlock), 0, st, L.md, L.tn, parity,
+                       (double)1.1f, output);
+    OR_HIP(hipGetLastError());
+    return OR_OK;
+  }
   if (L.nth > 0) {
     if (L.vh >= 2) or_ilp_elements(0, fp64, L.vh - 2, st, L.md, L.th, L.nth, po, L.eh);
     else launch_hex<R, S>(L.vh, st, L, po);
@@ -3039,10 +3120,25 @@ int or_batch_run(or_batch *b, int64_t ncycles) {
     L[c].tq = b->tiles[c][1]; L[c].ntq = b->nt[c][1]; L[c].vq = b->var[c][1];
     L[c].tn = b->tiles[c][2]; L[c].ntn = b->nt[c][2];
   }
+  // members of both forms and default variants: one element and one node launch for all of them
+  const bool both = L[0].ntn > 0 && L[1].ntn > 0 && !b->var[0][0] && !b->var[0][1] && !b->var[1][0] && !b->var[1][1];
+  ElemLists E{};
+  for (int c = 0; c < 2; ++c) {
+    E.t[2 * c + kFamQ4] = L[c].tq; E.n[2 * c + kFamQ4] = L[c].ntq;
+    E.t[2 * c + kFamHex] = L[c].th; E.n[2 * c + kFamHex] = L[c].nth;
+  }
+  const dim3 ge((unsigned)(E.n[0] + E.n[1] + E.n[2] + E.n[3])), gn((unsigned)(L[0].ntn + L[1].ntn));
   for (int64_t k = 0; k < ncycles; ++k) {
     const int p = (int)(b->parity & 1);
-    if ((rc = launch_cycle<double, double>(b->stream, L[0], p, nullptr, nullptr))) return rc;
-    if ((rc = launch_cycle<float, float>(b->stream, L[1], p, nullptr, nullptr))) return rc;
+    if (both) {
+      if (ge.x > 0) hipLaunchKernelGGL((k_elements<15, false>), ge, dim3(kTile), 0, b->stream, (const ModelDev *)b->md, E, p);
+      hipLaunchKernelGGL(k_node_update_both, gn, dim3(kBlock), 0, b->stream, (const ModelDev *)b->md, L[0].tn,
+                         L[0].ntn, L[1].tn, p, (double)1.1f);
+      OR_HIP(hipGetLastError());
+    } else {
+      if ((rc = launch_cycle<double, double>(b->stream, L[0], p, nullptr, nullptr))) return rc;
+      if ((rc = launch_cycle<float, float>(b->stream, L[1], p, nullptr, nullptr))) return rc;
+    }
     b->parity ^= 1;
     b->cycles += 1;
   }
