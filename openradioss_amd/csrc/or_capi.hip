@@ -447,16 +447,10 @@ __device__ __forceinline__ void hex_tile(const ModelDev &M, int64_t first, int p
   const int64_t i = first + threadIdx.x;
   const bool active = i < e.ne;
   const int64_t ic = active ? i : e.ne - 1;
-  // node ids first (vector loads return in order, and the gather waits for these), then the
-  // copies to LDS, in flight with the gather
   // the split form stages its element state through LDS; the FP64 chain, bound by its
   // arithmetic at two waves per SIMD, reads it from HBM after the kinematics (staged, it took
   // 15.2 us against 14.5 at 32,000 elements, and the same at 512,000)
   constexpr bool kStage = sizeof(S) == 4;
-  int32_t nc[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) nc[k] = e.conn[(int64_t)k * e.ne + ic];
-  __asm__ __volatile__("" ::: "memory");
   if constexpr (kStage) {
     const gptr<const S> src[12] = {e.sig,          e.sig + e.ne,     e.sig + 2 * e.ne, e.sig + 3 * e.ne,
                                    e.sig + 4 * e.ne, e.sig + 5 * e.ne, e.eint,           e.rho,
@@ -464,6 +458,10 @@ __device__ __forceinline__ void hex_tile(const ModelDev &M, int64_t first, int p
 #pragma unroll
     for (int a = 0; a < 12; ++a) stage_word<S>(sh.rows, a, src[a], first, e.ne);
   }
+  int32_t nc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) nc[k] = e.conn[(int64_t)k * e.ne + ic];
+  __asm__ __volatile__("" ::: "memory");
   TileAssembly<S, kHexRowWords, 8> ta;
   ta.range(M.hfr_start, first / kTile);
   const R DT1 = R(time_dt2(ts + parity));
@@ -634,7 +632,7 @@ __device__ __forceinline__ void q4_tile(const ModelDev &M, int64_t first, int pa
   const int64_t i = first + threadIdx.x;
   const bool active = i < q.ne;
   const int64_t ic = active ? i : q.ne - 1;
-  int32_t nc[4]; // node ids first, as in hex_tile
+  int32_t nc[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nc[k] = q.conn[(int64_t)k * q.ne + ic];
   __asm__ __volatile__("" ::: "memory");
@@ -813,43 +811,81 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   unsigned long long *dtmin = M.dtmin;
   const double dtmx = M.dtmx;
   const int64_t n = (int64_t)tl.first + threadIdx.x;
-  const DevTime prev = load_time(ts + parity);
   const bool in_range = n < nd.nn;
-  // ASSPAR4: rows of this node in skyline order (solids, then shells), from zero: the
-  // prefix the element tiles summed, then the rest rows in order
-  double ax = 0.0, ay = 0.0, az = 0.0, rx = 0.0, ry = 0.0, rz = 0.0;
-  int32_t dh = 0;
-  if (nd.deg_h && in_range) {
-    dh = to_global(nd.deg_h)[n];
-    if (dh > 0) {
-      const gptr<const double> p = to_global(nd.pre_h) + 3 * n;
-      ax = p[0]; ay = p[1]; az = p[2];
-      const gptr<const int32_t> rs = to_global(nd.rs_h);
-      const int32_t r1 = rs[n + 1];
-      for (int32_t r = rs[n]; r < r1; ++r) {
-        const gptr<const S> w = rowh + (int64_t)r * kHexRowWords;
-        ax = ax + double(w[0]); ay = ay + double(w[1]); az = az + double(w[2]);
-      }
-    }
+  const int64_t m = in_range ? n : nd.nn - 1;
+  // A small model's update is a chain of memory round trips (it fits in L2, one wave a SIMD), so
+  // everything that needs no other load is asked for first: the scalars, the node's records, its
+  // row counts, its hex prefix (unused when it has no hex rows).  37,000 nodes: 6.8 us between
+  // events where the loads stood at their uses and the rows came one by one 7.4; 690,000
+  // nodes, where bandwidth bounds it (4.6 TB/s): 39 and 40.  80 registers, six waves a SIMD;
+  // eight waves (64 registers) spill and take 69.
+  const DevTime prev = load_time(ts + parity);
+  const unsigned long long dt2t = to_global<const unsigned long long>(dtmin)[parity];
+  const gptr<v2d> p = (gptr<v2d>)to_global(nd.xv + 6 * m);
+  const v2d pa = p[0], pb = p[1], pc = p[2];
+  const gptr<double> dd = to_global(nd.d) + 3 * m;
+  const double d0 = dd[0], d1 = dd[1], d2 = dd[2];
+  const double msn = to_global(nd.ms)[m];
+  const int32_t code = to_global(nd.code)[m];
+  int32_t dh = 0, dq = 0, h0 = 0, h1 = 0, q0 = 0, q1 = 0;
+  double px = 0.0, py = 0.0, pz = 0.0;
+  if (nd.deg_h) {
+    dh = to_global(nd.deg_h)[m];
+    h0 = to_global(nd.rs_h)[m]; h1 = to_global(nd.rs_h)[m + 1];
+    const gptr<const double> q = to_global(nd.pre_h) + 3 * m;
+    px = q[0]; py = q[1]; pz = q[2];
   }
-  bool rot = false; // node carries rotational DOF work this cycle
-  if (nd.deg_q && in_range) {
-    const int32_t dq = to_global(nd.deg_q)[n];
-    rot = dq > 0;
-    if (dq > 0) {
-      if (dh == 0) { // the node's sum starts with its shell rows: their prefix
-        const gptr<const v2d> p = (gptr<const v2d>)(to_global(nd.pre_q) + 6 * n);
-        const v2d p0 = p[0], p1 = p[1], p2 = p[2];
-        ax = p0.x; ay = p0.y; az = p1.x; rx = p1.y; ry = p2.x; rz = p2.y;
-      }
-      const gptr<const int32_t> rs = to_global(nd.rs_q);
-      const int32_t r1 = rs[n + 1];
-      for (int32_t r = rs[n]; r < r1; ++r) {
-        const gptr<const S> w = rowq + (int64_t)r * kQ4RowWords;
-        ax = ax + double(w[0]); ay = ay + double(w[1]); az = az + double(w[2]);
-        rx = rx + double(w[3]); ry = ry + double(w[4]); rz = rz + double(w[5]);
-      }
+  if (nd.deg_q) {
+    dq = to_global(nd.deg_q)[m];
+    q0 = to_global(nd.rs_q)[m]; q1 = to_global(nd.rs_q)[m + 1];
+  }
+  // A node without shell rows and without rotational BCs has AR = 0, so VELOCITY leaves
+  // its VR as it is: its VR and IN are not touched.
+  bool rot = nd.vr && (dq > 0 || (code & (kRX | kRY | kRZ)));
+  double wx = 0.0, wy = 0.0, wz = 0.0, inn = 0.0;
+  gptr<v2d> pr = nullptr;
+  if (rot) {
+    inn = to_global(nd.in)[m];
+    pr = (gptr<v2d>)to_global(nd.vr + 4 * m);
+    const v2d r0 = pr[0], r1 = pr[1];
+    wx = r0.x; wy = r0.y; wz = r1.x;
+  }
+  // ASSPAR4: rows of this node in skyline order (solids, then shells), from zero: the
+  // prefix the element tiles summed, then the rest rows in order, some of them in flight at once
+  double ax = 0.0, ay = 0.0, az = 0.0, rx = 0.0, ry = 0.0, rz = 0.0;
+  if (dh > 0) { ax = px; ay = py; az = pz; }
+  if (dq > 0 && dh == 0) { // the node's sum starts with its shell rows: their prefix
+    const gptr<const v2d> q = (gptr<const v2d>)(to_global(nd.pre_q) + 6 * m);
+    const v2d p0 = q[0], p1 = q[1], p2 = q[2];
+    ax = p0.x; ay = p0.y; az = p1.x; rx = p1.y; ry = p2.x; rz = p2.y;
+  }
+  constexpr int kHexAhead = 4, kQ4Ahead = 3;
+  for (int32_t r = h0; r < h1; r += kHexAhead) {
+    S w[kHexAhead][kHexRowWords];
+#pragma unroll
+    for (int k = 0; k < kHexAhead; ++k) {
+      const gptr<const S> q = rowh + (int64_t)(r + k < h1 ? r + k : r) * kHexRowWords;
+#pragma unroll
+      for (int c = 0; c < kHexRowWords; ++c) w[k][c] = q[c];
     }
+#pragma unroll
+    for (int k = 0; k < kHexAhead; ++k)
+      if (r + k < h1) { ax = ax + double(w[k][0]); ay = ay + double(w[k][1]); az = az + double(w[k][2]); }
+  }
+  for (int32_t r = q0; r < q1; r += kQ4Ahead) {
+    S w[kQ4Ahead][kQ4RowWords];
+#pragma unroll
+    for (int k = 0; k < kQ4Ahead; ++k) {
+      const gptr<const S> q = rowq + (int64_t)(r + k < q1 ? r + k : r) * kQ4RowWords;
+#pragma unroll
+      for (int c = 0; c < kQ4RowWords; ++c) w[k][c] = q[c];
+    }
+#pragma unroll
+    for (int k = 0; k < kQ4Ahead; ++k)
+      if (r + k < q1) {
+        ax = ax + double(w[k][0]); ay = ay + double(w[k][1]); az = az + double(w[k][2]);
+        rx = rx + double(w[k][3]); ry = ry + double(w[k][4]); rz = rz + double(w[k][5]);
+      }
   }
   if (prev.done) {
     // a stopped model keeps its state; its scalars are carried to the other parity
@@ -861,8 +897,7 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   }
   // DT2 pipeline (resol.F:2721-2722, 2826, 6125-6129, 6352, 6494-6497)
   const double DT1 = prev.dt2;
-  const double DT2 = dt2_pipeline(bitsd(to_global<const unsigned long long>(dtmin)[parity]), prev.dt2old,
-                                  dt_growth, dtmx);
+  const double DT2 = dt2_pipeline(bitsd(dt2t), prev.dt2old, dt_growth, dtmx);
   const double DT12 = (1.0 / 2.0) * (DT1 + DT2);
   if (n == 0) {
     DevTime nx;
@@ -880,22 +915,8 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   }
   if (!in_range) return;
   // ACCELE (accele.F:65-80, 97-109)
-  const double msn = to_global(nd.ms)[n];
   accele3(ax, ay, az, msn);
-  const int32_t code = to_global(nd.code)[n];
-  // A node without shell rows and without rotational BCs has AR = 0, so VELOCITY leaves
-  // its VR as it is: its VR and IN are not touched.
-  rot = rot || (code & (kRX | kRY | kRZ));
-  double wx = 0.0, wy = 0.0, wz = 0.0;
-  gptr<v2d> pr = nullptr;
-  if (nd.vr && rot) {
-    accele3(rx, ry, rz, to_global(nd.in)[n]);
-    pr = (gptr<v2d>)to_global(nd.vr + 4 * n);
-    const v2d r0 = pr[0], r1 = pr[1];
-    wx = r0.x; wy = r0.y; wz = r1.x;
-  }
-  const gptr<v2d> p = (gptr<v2d>)to_global(nd.xv + 6 * n);
-  const v2d pa = p[0], pb = p[1], pc = p[2];
+  if (rot) accele3(rx, ry, rz, inn);
   double x = pa.x, y = pa.y, z = pb.x, vx = pb.y, vy = pc.x, vz = pc.y;
   if (code) {
     // the node's external work (WFEXT) accumulates in wext[n] when its DOFs are imposed
@@ -918,7 +939,7 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
     ke[n] = (ux * ux + uy * uy + uz * uz) * (1.0 / 2.0) * msn;
     double kr = 0.0;
     if (nd.vr) {
-      double qx = wx, qy = wy, qz = wz, inn = 0.0;
+      double qx = wx, qy = wy, qz = wz;
       if (!pr) { // rotational work skipped: AR = 0, VR as stored
         const gptr<const v2d> q = (gptr<const v2d>)to_global(nd.vr + 4 * n);
         const v2d q0 = q[0], q1 = q[1];
@@ -964,11 +985,10 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
     pr[1] = v2d{wz, 0.0};
   }
   // DEPLA (displacement.F:108-118, IRESP=0 form in FP64)
-  const gptr<double> dd = to_global(nd.d) + 3 * n;
   double vdt;
-  vdt = DT2 * vx; dd[0] = dd[0] + vdt; x = x + vdt;
-  vdt = DT2 * vy; dd[1] = dd[1] + vdt; y = y + vdt;
-  vdt = DT2 * vz; dd[2] = dd[2] + vdt; z = z + vdt;
+  vdt = DT2 * vx; dd[0] = d0 + vdt; x = x + vdt;
+  vdt = DT2 * vy; dd[1] = d1 + vdt; y = y + vdt;
+  vdt = DT2 * vz; dd[2] = d2 + vdt; z = z + vdt;
   p[0] = v2d{x, y};
   p[1] = v2d{z, vx};
   p[2] = v2d{vy, vz};
