@@ -293,7 +293,7 @@ int or_batch_active(or_batch *b, int32_t *nactive);
 /* ---- launch variants of the element kernels and their autotuning ----
  * No counterpart in the reference.  Variant v (0..3) of the hex (family 0) or shell
  * (family 1) kernel sets the register budget it is compiled for (two waves per SIMD for
- * even v, three for odd v) and the compiler's instruction scheduler (default for v < 2,
+ * even v, three for odd v; FP64 two in both) and the compiler's instruction scheduler (default for v < 2,
  * ILP-first for v >= 2); every workgroup is one tile of 256 elements.  All variants
  * compute bit-identical results.  The autotuners time cycles_per_variant real
  * cycles per candidate (the models advance meanwhile) and keep the fastest:
