@@ -6,6 +6,7 @@
 //                  (both fold their element time steps into one device word with an
 //                  integer atomicMin on the FP64 bit pattern: min is exact, so the
 //                  result does not depend on block order)
+//   k_elements   : both, in one launch, when a model or batch has more than one family or form
 //   k_node_update: ASSPAR4 fixed-order segmented sum per node (hex rows, then Q4 rows,
 //                  the FILLCNE order), DT2 pipeline, ACCELE, BCS10, FIXVEL, VELOCITY,
 //                  DEPLA; thread 0 advances the cycle scalars (double-buffered by parity)
@@ -3033,7 +3034,7 @@ int or_model_footprint(const or_model *m, int64_t *bytes) {
 
 // ============================================================== group drop-ins
 namespace {
-// Device staging of one group call: every buffer allocated, copied, freed here.
+// Device buffers of one diagnostic call: allocated, copied and freed here.
 struct Stage {
   std::vector<void *> ptrs;
   hipError_t e = hipSuccess;
