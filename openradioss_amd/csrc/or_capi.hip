@@ -812,8 +812,10 @@ __host__ __device__ __forceinline__ double dt2_pipeline(double dt2t, double dt2o
 }
 
 // ---------------------------------------------------------------- node kernel
-// Block b of a launch's list, or of the only model's nodes.
-template <typename S>
+// Block b of a launch's list, or of the only model's nodes.  FIRST: everything that needs no other
+// load is asked for at the start and the rest rows come several at a time; otherwise every load stands
+// at its use (node_first chooses).  Both add the same values in the same order.
+template <typename S, bool FIRST>
 __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const Tile *__restrict__ tiles, int32_t b,
                                           int parity, double dt_growth, int output) {
   const Tile tl = tiles ? tiles[b] : Tile{0, b * kBlock};
@@ -827,53 +829,60 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   const int64_t n = (int64_t)tl.first + threadIdx.x;
   const bool in_range = n < nd.nn;
   const int64_t m = in_range ? n : nd.nn - 1;
-  // A small model's update is a chain of memory round trips (it fits in L2, one wave a SIMD), so
-  // everything that needs no other load is asked for first: the scalars, the node's records, its
-  // row counts, its hex prefix (unused when it has no hex rows).  37,000 nodes: 6.8 us between
-  // events where the loads stood at their uses and the rows came one by one 7.4; 690,000
-  // nodes, where bandwidth bounds it (4.6 TB/s): 39 and 40.  80 registers, six waves a SIMD;
-  // eight waves (64 registers) spill and take 69.
   const DevTime prev = load_time(ts + parity);
-  const unsigned long long dt2t = to_global<const unsigned long long>(dtmin)[parity];
-  const gptr<v2d> p = (gptr<v2d>)to_global(nd.xv + 6 * m);
-  const v2d pa = p[0], pb = p[1], pc = p[2];
-  const gptr<double> dd = to_global(nd.d) + 3 * m;
-  const double d0 = dd[0], d1 = dd[1], d2 = dd[2];
-  const double msn = to_global(nd.ms)[m];
-  const int32_t code = to_global(nd.code)[m];
-  int32_t dh = 0, dq = 0, h0 = 0, h1 = 0, q0 = 0, q1 = 0;
+  unsigned long long dt2t;
+  v2d pa, pb, pc;
+  double d0, d1, d2, msn;
+  int32_t code, dh = 0, dq = 0, h0 = 0, h1 = 0, q0 = 0, q1 = 0;
   double px = 0.0, py = 0.0, pz = 0.0;
-  if (nd.deg_h) {
-    dh = to_global(nd.deg_h)[m];
-    h0 = to_global(nd.rs_h)[m]; h1 = to_global(nd.rs_h)[m + 1];
-    const gptr<const double> q = to_global(nd.pre_h) + 3 * m;
-    px = q[0]; py = q[1]; pz = q[2];
-  }
-  if (nd.deg_q) {
-    dq = to_global(nd.deg_q)[m];
-    q0 = to_global(nd.rs_q)[m]; q1 = to_global(nd.rs_q)[m + 1];
-  }
-  // A node without shell rows and without rotational BCs has AR = 0, so VELOCITY leaves
-  // its VR as it is: its VR and IN are not touched.
-  bool rot = nd.vr && (dq > 0 || (code & (kRX | kRY | kRZ)));
+  bool rot = false;
   double wx = 0.0, wy = 0.0, wz = 0.0, inn = 0.0;
   gptr<v2d> pr = nullptr;
-  if (rot) {
-    inn = to_global(nd.in)[m];
-    pr = (gptr<v2d>)to_global(nd.vr + 4 * m);
-    const v2d r0 = pr[0], r1 = pr[1];
-    wx = r0.x; wy = r0.y; wz = r1.x;
+  if constexpr (FIRST) {
+    dt2t = to_global<const unsigned long long>(dtmin)[parity];
+    const gptr<const v2d> p = (gptr<const v2d>)to_global(nd.xv + 6 * m);
+    pa = p[0]; pb = p[1]; pc = p[2];
+    const gptr<const double> dd = to_global(nd.d) + 3 * m;
+    d0 = dd[0]; d1 = dd[1]; d2 = dd[2];
+    msn = to_global(nd.ms)[m];
+    code = to_global(nd.code)[m];
+    if (nd.deg_h) {
+      dh = to_global(nd.deg_h)[m];
+      h0 = to_global(nd.rs_h)[m]; h1 = to_global(nd.rs_h)[m + 1];
+      const gptr<const double> q = to_global(nd.pre_h) + 3 * m; // unused when the node has no hex rows
+      px = q[0]; py = q[1]; pz = q[2];
+    }
+    if (nd.deg_q) {
+      dq = to_global(nd.deg_q)[m];
+      q0 = to_global(nd.rs_q)[m]; q1 = to_global(nd.rs_q)[m + 1];
+    }
+    // A node without shell rows and without rotational BCs has AR = 0, so VELOCITY leaves
+    // its VR as it is: its VR and IN are not touched.
+    rot = nd.vr && (dq > 0 || (code & (kRX | kRY | kRZ)));
+    if (rot) {
+      inn = to_global(nd.in)[m];
+      pr = (gptr<v2d>)to_global(nd.vr + 4 * m);
+      const v2d r0 = pr[0], r1 = pr[1];
+      wx = r0.x; wy = r0.y; wz = r1.x;
+    }
+  } else if (nd.deg_h && in_range) {
+    dh = to_global(nd.deg_h)[n];
+    if (dh > 0) {
+      const gptr<const double> q = to_global(nd.pre_h) + 3 * n;
+      px = q[0]; py = q[1]; pz = q[2];
+      h0 = to_global(nd.rs_h)[n]; h1 = to_global(nd.rs_h)[n + 1];
+    }
   }
   // ASSPAR4: rows of this node in skyline order (solids, then shells), from zero: the
-  // prefix the element tiles summed, then the rest rows in order, some of them in flight at once
+  // prefix the element tiles summed, then the rest rows in order
   double ax = 0.0, ay = 0.0, az = 0.0, rx = 0.0, ry = 0.0, rz = 0.0;
   if (dh > 0) { ax = px; ay = py; az = pz; }
-  if (dq > 0 && dh == 0) { // the node's sum starts with its shell rows: their prefix
+  if (FIRST && dq > 0 && dh == 0) { // the node's sum starts with its shell rows: their prefix
     const gptr<const v2d> q = (gptr<const v2d>)(to_global(nd.pre_q) + 6 * m);
     const v2d p0 = q[0], p1 = q[1], p2 = q[2];
     ax = p0.x; ay = p0.y; az = p1.x; rx = p1.y; ry = p2.x; rz = p2.y;
   }
-  constexpr int kHexAhead = 4, kQ4Ahead = 3;
+  constexpr int kHexAhead = FIRST ? 4 : 1, kQ4Ahead = FIRST ? 3 : 1; // rest rows in flight at once
   for (int32_t r = h0; r < h1; r += kHexAhead) {
     S w[kHexAhead][kHexRowWords];
 #pragma unroll
@@ -885,6 +894,19 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
 #pragma unroll
     for (int k = 0; k < kHexAhead; ++k)
       if (r + k < h1) { ax = ax + double(w[k][0]); ay = ay + double(w[k][1]); az = az + double(w[k][2]); }
+  }
+  if constexpr (!FIRST) {
+    if (nd.deg_q && in_range) {
+      dq = to_global(nd.deg_q)[n];
+      if (dq > 0) {
+        if (dh == 0) {
+          const gptr<const v2d> q = (gptr<const v2d>)(to_global(nd.pre_q) + 6 * n);
+          const v2d p0 = q[0], p1 = q[1], p2 = q[2];
+          ax = p0.x; ay = p0.y; az = p1.x; rx = p1.y; ry = p2.x; rz = p2.y;
+        }
+        q0 = to_global(nd.rs_q)[n]; q1 = to_global(nd.rs_q)[n + 1];
+      }
+    }
   }
   for (int32_t r = q0; r < q1; r += kQ4Ahead) {
     S w[kQ4Ahead][kQ4RowWords];
@@ -910,6 +932,7 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
     return;
   }
   // DT2 pipeline (resol.F:2721-2722, 2826, 6125-6129, 6352, 6494-6497)
+  if constexpr (!FIRST) dt2t = to_global<const unsigned long long>(dtmin)[parity];
   const double DT1 = prev.dt2;
   const double DT2 = dt2_pipeline(bitsd(dt2t), prev.dt2old, dt_growth, dtmx);
   const double DT12 = (1.0 / 2.0) * (DT1 + DT2);
@@ -929,8 +952,21 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   }
   if (!in_range) return;
   // ACCELE (accele.F:65-80, 97-109)
+  if constexpr (!FIRST) msn = to_global(nd.ms)[n];
   accele3(ax, ay, az, msn);
+  if constexpr (!FIRST) {
+    code = to_global(nd.code)[n];
+    rot = nd.vr && (dq > 0 || (code & (kRX | kRY | kRZ)));
+    if (rot) {
+      inn = to_global(nd.in)[n];
+      pr = (gptr<v2d>)to_global(nd.vr + 4 * n);
+      const v2d r0 = pr[0], r1 = pr[1];
+      wx = r0.x; wy = r0.y; wz = r1.x;
+    }
+  }
   if (rot) accele3(rx, ry, rz, inn);
+  const gptr<v2d> p = (gptr<v2d>)to_global(nd.xv + 6 * n);
+  if constexpr (!FIRST) { pa = p[0]; pb = p[1]; pc = p[2]; }
   double x = pa.x, y = pa.y, z = pb.x, vx = pb.y, vy = pc.x, vz = pc.y;
   if (code) {
     // the node's external work (WFEXT) accumulates in wext[n] when its DOFs are imposed
@@ -999,6 +1035,8 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
     pr[1] = v2d{wz, 0.0};
   }
   // DEPLA (displacement.F:108-118, IRESP=0 form in FP64)
+  const gptr<double> dd = to_global(nd.d) + 3 * n;
+  if constexpr (!FIRST) { d0 = dd[0]; d1 = dd[1]; d2 = dd[2]; }
   double vdt;
   vdt = DT2 * vx; dd[0] = d0 + vdt; x = x + vdt;
   vdt = DT2 * vy; dd[1] = d1 + vdt; y = y + vdt;
@@ -1008,22 +1046,24 @@ __device__ __forceinline__ void node_tile(const ModelDev *__restrict__ md, const
   p[2] = v2d{vy, vz};
 }
 
-template <typename S>
+template <typename S, bool FIRST>
 __global__ __launch_bounds__(kBlock) void k_node_update(const ModelDev *__restrict__ md,
                                                         const Tile *__restrict__ tiles, int parity,
                                                         double dt_growth, int output) {
-  node_tile<S>(md, tiles, (int32_t)blockIdx.x, parity, dt_growth, output);
+  node_tile<S, FIRST>(md, tiles, (int32_t)blockIdx.x, parity, dt_growth, output);
 }
 
 // The node update of a batch with members of both forms, in one launch: n64 blocks of FP64
-// members, then those of the split form.
+// members, then those of the split form.  98 registers, four waves a SIMD; still the fastest at every
+// size (12 bars and tubes: 41.6 us a cycle against 45.6 in a launch for each form at 98,000 nodes, 110
+// and 115 at 515,000, 498 and 506 at 2,586,000, 1,508 and 1,515 at 8,072,000; held to five waves 1,513).
 __global__ __launch_bounds__(kBlock) void k_node_update_both(const ModelDev *__restrict__ md,
                                                              const Tile *__restrict__ t64, int32_t n64,
                                                              const Tile *__restrict__ t32, int parity,
                                                              double dt_growth) {
   const int32_t b = (int32_t)blockIdx.x;
-  if (b < n64) node_tile<double>(md, t64, b, parity, dt_growth, 0);
-  else node_tile<float>(md, t32, b - n64, parity, dt_growth, 0);
+  if (b < n64) node_tile<double, true>(md, t64, b, parity, dt_growth, 0);
+  else node_tile<float, true>(md, t32, b - n64, parity, dt_growth, 0);
 }
 
 // ---------------------------------------------------------------- energies (fixed-order)
@@ -2534,6 +2574,22 @@ static LaunchSet model_set(const or_model *m) {
 // 104.4), a batch of 12 bars and tubes in both forms 47.0 (103.2).
 static bool one_launch(const LaunchSet &L) { return L.nth > 0 && L.ntq > 0 && L.vh == 0 && L.vq == 0; }
 
+// Which form of the node update a launch of nb blocks takes.  A small model's update is a chain of
+// memory round trips (it fits in L2, one wave a SIMD), so its loads come first (76 registers, six waves
+// a SIMD; 70 and seven in the split form); a large one is bound by HBM and takes the loads at their uses
+// (64 registers, eight waves).  us at FP64 / split form, loads first against at their uses: 45,000
+// nodes 7.8 / 7.9 and 8.9 / 8.2; 373,000 21.3 / 20.0 and 22.6 / 20.4; 1,264,000 82 / 62 and 83 / 64;
+// 1,921,000 123 / 97 and 123 / 96; 2,771,000 172 / 140 and 172 / 134; 5,149,000 310 / 255 and 302 / 242
+// (4.4 TB/s).
+static bool node_first(int64_t nb) { return nb < 8192; }
+
+template <typename S> static void launch_nodes(hipStream_t st, const LaunchSet &L, int parity, int output) {
+  const dim3 g((unsigned)L.ntn);
+  const double growth = (double)1.1f;
+  if (node_first(L.ntn)) hipLaunchKernelGGL((k_node_update<S, true>), g, dim3(kBlock), 0, st, L.md, L.tn, parity, growth, output);
+  else hipLaunchKernelGGL((k_node_update<S, false>), g, dim3(kBlock), 0, st, L.md, L.tn, parity, growth, output);
+}
+
 template <typename R, typename S>
 static int launch_cycle(hipStream_t st, const LaunchSet &L, int parity, hipEvent_t after_hex, hipEvent_t after_q4,
                         int output = 0) {
@@ -2549,8 +2605,7 @@ static int launch_cycle(hipStream_t st, const LaunchSet &L, int parity, hipEvent
     if (L.eh || L.eq) hipLaunchKernelGGL((k_elements<mask, true>), g, dim3(kTile), 0, st, L.md, E, po);
     else hipLaunchKernelGGL((k_elements<mask, false>), g, dim3(kTile), 0, st, L.md, E, po);
     OR_HIP(hipGetLastError());
-    hipLaunchKernelGGL((k_node_update<S>), dim3((unsigned)L.ntn), dim3(kBlock), 0, st, L.md, L.tn, parity,
-                       (double)1.1f, output);
+    launch_nodes<S>(st, L, parity, output);
     OR_HIP(hipGetLastError());
     return OR_OK;
   }
@@ -2567,8 +2622,7 @@ static int launch_cycle(hipStream_t st, const LaunchSet &L, int parity, hipEvent
   }
   if (after_q4) OR_HIP(hipEventRecord(after_q4, st));
   if (L.ntn > 0) {
-    hipLaunchKernelGGL((k_node_update<S>), dim3((unsigned)L.ntn), dim3(kBlock), 0, st, L.md, L.tn, parity,
-                       (double)1.1f, output);
+    launch_nodes<S>(st, L, parity, output);
     OR_HIP(hipGetLastError());
   }
   return OR_OK;
