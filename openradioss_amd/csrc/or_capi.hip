@@ -629,6 +629,16 @@ template <typename R, typename S> struct Q4IpIO {
   }
 };
 
+// The thread's element, formed again where it stands instead of held in registers from the tile's
+// start: two registers of the FP64 shells' 256, which else spill 12 bytes a lane (160,000 elastic shells
+// 47.7 us a cycle for 48.8; a kernel with scratch also starts 0.5 us later).  The FP64 hexes spill as
+// much but keep theirs: without it the 4,096,000 + 1,000,000 elements in one launch take 1,026 us for 1,004.
+__device__ __forceinline__ int64_t element_again(int64_t first) {
+  int t = threadIdx.x;
+  __asm__ __volatile__("" : "+v"(t));
+  return first + t;
+}
+
 // ---------------------------------------------------------------- Q4 element tile
 // The CFORC3 chain of one tile; threads past the last element as in hex_tile.
 template <typename R, typename S, bool EH>
@@ -642,9 +652,7 @@ __device__ __forceinline__ void q4_tile(const ModelDev &M, int64_t first, int pa
   const gptr<const double> xv = to_global<const double>(M.nd.xv);
   const gptr<const double> vr = to_global<const double>(M.nd.vr);
   const Q4Consts &c = M.qc;
-  const int64_t i = first + threadIdx.x;
-  const bool active = i < q.ne;
-  const int64_t ic = active ? i : q.ne - 1;
+  const int64_t ic = std::min<int64_t>(first + threadIdx.x, q.ne - 1);
   int32_t nc[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nc[k] = q.conn[(int64_t)k * q.ne + ic];
@@ -666,7 +674,7 @@ __device__ __forceinline__ void q4_tile(const ModelDev &M, int64_t first, int pa
   }
   Q4Elem<R> st;
   st.offg = R(q.offg[ic]); st.thk = R(q.thk[ic]); st.thke = R(q.thke[ic]); st.epsd = R(q.epsd[ic]);
-  Q4IpIO<R, S> io{q, ic, active && !stopped, c.npt};
+  Q4IpIO<R, S> io{q, ic, first + threadIdx.x < q.ne && !stopped, c.npt};
   Q4Out<R> o;
   // EH: the model keeps EHOUR (its own instantiation, so that the other keeps its registers)
   auto ehou_sink = [&](R v) {
@@ -681,6 +689,8 @@ __device__ __forceinline__ void q4_tile(const ModelDev &M, int64_t first, int pa
   };
   q4_element<R>(xg, yg, zg, vl, vrl, nc[2] == nc[3], st, c, DT1, io, nload, o, ehou_sink, chain_tab<R>(sh.tab));
   if (stopped) return; // uniform over the workgroup
+  const int64_t i = element_again(first);
+  const bool active = i < q.ne;
   if (active) {
     q.offg[i] = S(st.offg); q.thk[i] = S(st.thk); q.epsd[i] = S(st.epsd);
     if (output && M.dtel_q) to_global(M.dtel_q)[i] = o.dt;

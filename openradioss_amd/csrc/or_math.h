@@ -240,7 +240,9 @@ __host__ __device__ inline double or_log(double x, const T tab = T{}) {
   if (!(x >= kMinNormal && x <= kMaxFinite)) return log(x);
   double f;
   if (kTryFast && try_log(x, f, tab)) return f;
-  dd l = log_dd(x, tab);
+  // the rare path reads the constant arrays: through the shells' copy in LDS it costs them registers
+  // that spill (28 bytes a lane)
+  dd l = log_dd(x);
   return l.hi + l.lo;
 }
 
