@@ -292,12 +292,14 @@ int or_batch_active(or_batch *b, int32_t *nactive);
 
 /* ---- launch variants of the element kernels and their autotuning ----
  * No counterpart in the reference.  Variant v (0..3) of the hex (family 0) or shell
- * (family 1) kernel sets the register budget it is compiled for (two waves per SIMD for
- * even v, three for odd v; FP64 two in both) and the compiler's instruction scheduler (default for v < 2,
- * ILP-first for v >= 2); every workgroup is one tile of 256 elements.  All variants
- * compute bit-identical results.  The autotuners time cycles_per_variant real
- * cycles per candidate (the models advance meanwhile) and keep the fastest:
- * chosen[family] for a model, chosen[2*precision + family] for a batch. */
+ * (family 1) kernel sets the compiler's instruction scheduler (default for v < 2, ILP-first
+ * for v >= 2) and the register budget it is compiled for (two waves per SIMD for even v, three
+ * for odd v).  Where both budgets give one kernel an odd v stands for the even one below it:
+ * FP64, and the split form's hexes with v = 1.  Every workgroup is one tile of 256 elements.
+ * All variants compute bit-identical results.  Families of default variants share one launch.
+ * The autotuners time 4 * cycles_per_variant real cycles a family (the models advance
+ * meanwhile), the joint launch among the candidates, and keep the fastest; the default unless
+ * another is 2 % faster: chosen[family] for a model, chosen[2*precision + family] for a batch. */
 int or_model_set_variant(or_model *m, int family, int variant);
 int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]);
 int or_batch_autotune(or_batch *b, int32_t cycles_per_variant, int32_t chosen[4]);

@@ -57,17 +57,25 @@ int fail(int code, const std::string &msg) {
 constexpr int kBlock = 256;
 constexpr double kNoEnd = 1.0e300; // end time of a model advanced by or_model_run
 
-// Launch variants of the element kernels.  Variant v picks the minimum number of waves
-// per SIMD the register allocation is built for (split form: two for even v, three for odd
-// v; FP64: two, since three spill to scratch; a wave's register budget is 512 / waves VGPRs
-// and AGPRs together) and the instruction scheduler (default for v < 2, ILP-first for v >= 2).
+// Launch variants of the element kernels.  Variant v picks the instruction scheduler (default
+// for v < 2, ILP-first for v >= 2) and, in the split form, the minimum number of waves per SIMD the
+// register allocation is built for (two for even v, three for odd v; a wave's register budget is 512 /
+// waves VGPRs and AGPRs together).  Where both budgets give the same kernel, the odd variant is
+// the even one: FP64 (three waves spill 316 bytes a lane and take twice the time) and the split
+// form's hexes under the default scheduler (156 registers, three waves in either).
 // Every element workgroup is one tile of kTile elements, the unit of the LDS assembly.
 // Every variant runs the same arithmetic, so the choice (or_model_set_variant,
 // or_model_autotune, or_batch_autotune) changes speed only, never a result bit.
 constexpr int kVariants = 4;
 constexpr int kTile = orasm::kTile;
 static_assert(kTile == kBlock, "element tiles and node blocks share the workgroup size");
-template <typename R> constexpr int variant_waves(int v) { return sizeof(R) == 8 ? 2 : 2 + (v & 1); }
+// The variant that is built for variant v of a family (0: hexes, 1: shells).
+constexpr int built_variant(bool fp64, int family, int v) {
+  if (fp64) return v & 2;
+  return family == 0 && v == 1 ? 0 : v;
+}
+// Waves per SIMD of built variant v.
+constexpr int variant_waves(bool fp64, int v) { return fp64 ? 2 : 2 + (v & 1); }
 
 // MSTOP codes (include/or_gpu.h): an element's non-positive Jacobian, a time step <= 0
 constexpr int32_t kMstopJacobian = 1, kMstopTimeStep = 2;
@@ -1844,7 +1852,7 @@ struct or_model {
   ModelDev *dev = nullptr;
   bool dev_dirty = true;
   int32_t nt_h = 0, nt_q = 0, nt_n = 0;
-  int var_h = 0, var_q = 0;            // element kernel variants
+  int var_h = 0, var_q = 0;            // element kernel variants, as built
   or_batch *batch = nullptr;           // set while the model belongs to a batch
   // timing
   bool timing = false;
@@ -1865,7 +1873,7 @@ struct or_batch {
   ModelDev *md = nullptr;          // device array of the slots' kernel views
   int64_t md_cap = 0;
   Tile *tiles[2][3] = {};          // [precision][hex, q4, node]
-  int var[2][2] = {};              // element kernel variants [precision][hex, q4]
+  int var[2][2] = {};              // element kernel variants, as built [precision][hex, q4]
   int32_t nt[2][3] = {};
   int64_t tcap[2][3] = {};
   bool dirty = true;
@@ -2513,15 +2521,22 @@ struct LaunchSet {
   const ModelDev *md = nullptr;
   const Tile *th = nullptr, *tq = nullptr, *tn = nullptr;
   int32_t nth = 0, ntq = 0, ntn = 0;
-  int vh = 0, vq = 0; // element kernel variants (their block sizes match th / tq)
+  int vh = 0, vq = 0; // element kernel variants, as built
   bool eh = false, eq = false; // the set keeps EHOUR (hexes, shells): one model with a time history
 };
 
-// v & 1 selects the register budget (2 or 3 waves per SIMD); the caller routes v >= 2 to
-// the unit built with the ILP-first scheduler.
+// v & 1 selects the register budget; the caller routes v >= 2 to the unit built with the
+// ILP-first scheduler.
+#ifdef OR_ILP_TU
+constexpr int kUnitFirst = 2; // this unit's first variant
+#else
+constexpr int kUnitFirst = 0;
+#endif
 template <typename R, typename S, bool EH>
 static void launch_hex_eh(int v, hipStream_t st, const LaunchSet &L, int parity) {
-  constexpr int W0 = variant_waves<R>(0), W1 = variant_waves<R>(1);
+  constexpr bool fp64 = sizeof(R) == 8;
+  constexpr int W0 = variant_waves(fp64, built_variant(fp64, 0, kUnitFirst)),
+                W1 = variant_waves(fp64, built_variant(fp64, 0, kUnitFirst + 1));
   const dim3 g((unsigned)L.nth);
   if ((v & 1) == 0) hipLaunchKernelGGL((k_hex_forces<R, S, kTile, W0, EH>), g, dim3(kTile), 0, st, L.md, L.th, parity);
   else hipLaunchKernelGGL((k_hex_forces<R, S, kTile, W1, EH>), g, dim3(kTile), 0, st, L.md, L.th, parity);
@@ -2534,7 +2549,9 @@ static void launch_hex(int v, hipStream_t st, const LaunchSet &L, int parity) {
 
 template <typename R, typename S, bool EH>
 static void launch_q4_eh(int v, hipStream_t st, const LaunchSet &L, int parity) {
-  constexpr int W0 = variant_waves<R>(0), W1 = variant_waves<R>(1);
+  constexpr bool fp64 = sizeof(R) == 8;
+  constexpr int W0 = variant_waves(fp64, built_variant(fp64, 1, kUnitFirst)),
+                W1 = variant_waves(fp64, built_variant(fp64, 1, kUnitFirst + 1));
   const dim3 g((unsigned)L.ntq);
   if ((v & 1) == 0) hipLaunchKernelGGL((k_q4_forces<R, S, kTile, W0, EH>), g, dim3(kTile), 0, st, L.md, L.tq, parity);
   else hipLaunchKernelGGL((k_q4_forces<R, S, kTile, W1, EH>), g, dim3(kTile), 0, st, L.md, L.tq, parity);
@@ -3608,19 +3625,72 @@ int or_batch_active(or_batch *b, int32_t *nactive) {
 // Kernel variants and their autotuning
 namespace {
 
-// Device time of `ncycles` cycles launched by `launch` on `st` (events around the loop).
+// Device time of `ncycles` cycles launched by `launch` on `st` (events around the loop).  Of several
+// cycles the first, which may have to load its kernels' code, is not in the time.
 template <typename F> int time_cycles(hipStream_t st, int ncycles, F launch, float &ms) {
   hipEvent_t e0, e1;
   OR_HIP(hipEventCreate(&e0));
   OR_HIP(hipEventCreate(&e1));
   int rc = OR_OK;
-  if (hipEventRecord(e0, st) != hipSuccess) rc = fail(OR_ERR_HIP, "hipEventRecord");
-  for (int k = 0; k < ncycles && rc == OR_OK; ++k) rc = launch();
+  const int untimed = ncycles > 1 ? 1 : 0;
+  for (int k = 0; k < ncycles && rc == OR_OK; ++k) {
+    if (k == untimed && hipEventRecord(e0, st) != hipSuccess) rc = fail(OR_ERR_HIP, "hipEventRecord");
+    if (rc == OR_OK) rc = launch();
+  }
   if (rc == OR_OK && (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                       hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
     rc = fail(OR_ERR_HIP, "event timing");
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  return rc;
+}
+
+// The variants of a model's (or a batch form's) families: trial(h, q, ms) runs cycles_per_variant
+// cycles with variants h and q.  The default pair, whose families share a launch, is measured
+// against pairs with a launch each: hexes' other variants, shells' with the best of those, the default
+// hexes with the best shells.  kVariants trials a family in all; those left over repeat the default and
+// the best other pair, whose shortest times count.  Another pair is taken only when it is 2 %
+// faster, which is what two measurements of one pair differ by.
+template <typename F> int tune_variants(bool fp64, bool has_hex, bool has_q4, F trial, int best[2]) {
+  constexpr float kNone = 1.0e30f;
+  float t[kVariants][kVariants];
+  for (auto &row : t) std::fill(std::begin(row), std::end(row), kNone);
+  int left = kVariants * ((has_hex ? 1 : 0) + (has_q4 ? 1 : 0));
+  int rc = OR_OK;
+  auto run = [&](int h, int q) {
+    if (rc != OR_OK || left == 0) return;
+    --left;
+    float ms = kNone;
+    rc = trial(h, q, ms);
+    t[h][q] = std::min(t[h][q], ms);
+  };
+  auto fastest_other = [&](int &h, int &q) { // of the pairs measured, the default one apart
+    h = q = 0;
+    float ms = kNone;
+    for (int a = 0; a < kVariants; ++a)
+      for (int b = 0; b < kVariants; ++b)
+        if ((a || b) && t[a][b] < ms) { h = a; q = b; ms = t[a][b]; }
+    return ms;
+  };
+  run(0, 0);
+  int h = 0, q = 0;
+  for (int v = 1; has_hex && v < kVariants; ++v)
+    if (built_variant(fp64, 0, v) == v) run(v, 0);
+  fastest_other(h, q);
+  const int hs = h;
+  for (int v = 1; has_q4 && v < kVariants; ++v)
+    if (built_variant(fp64, 1, v) == v) run(hs, v);
+  fastest_other(h, q);
+  if (has_hex && has_q4) run(0, q ? q : 2);
+  while (left > 0 && rc == OR_OK) {
+    run(0, 0);
+    fastest_other(h, q);
+    run(h, q);
+  }
+  const float ms = fastest_other(h, q);
+  const bool take = rc == OR_OK && ms < 0.98f * t[0][0];
+  best[0] = take ? h : 0;
+  best[1] = take ? q : 0;
   return rc;
 }
 
@@ -3631,7 +3701,7 @@ int or_model_set_variant(or_model *m, int family, int variant) {
   if (family < 0 || family > 1 || variant < 0 || variant >= kVariants) return fail(OR_ERR_ARG, "bad family / variant");
   OR_HIP(hipSetDevice(m->device));
   OR_HIP(quiesce(m));
-  (family == 0 ? m->var_h : m->var_q) = variant;
+  (family == 0 ? m->var_h : m->var_q) = built_variant(m->prec == OR_PREC_FP64, family, variant);
   return OR_OK;
 }
 
@@ -3645,26 +3715,24 @@ int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]
   OR_HIP(hipSetDevice(m->device));
   int rc = refresh_dev(m);
   if (rc) return rc;
-  for (int f = 0; f < 2; ++f) {
-    if ((f == 0 ? m->neh : m->neq) == 0) continue;
-    int best = 0;
-    float best_ms = 0.f;
-    for (int v = 0; v < kVariants; ++v) {
-      if ((rc = or_model_set_variant(m, f, v))) return rc;
-      const LaunchSet L = model_set(m);
-      float ms = 0.f;
-      auto one = [&]() -> int {
-        const int p = (int)(m->parity & 1);
-        int r = (m->prec == OR_PREC_FP64) ? launch_cycle<double, double>(m->stream, L, p, nullptr, nullptr)
-                                          : launch_cycle<float, float>(m->stream, L, p, nullptr, nullptr);
-        m->parity ^= 1;
-        return r;
-      };
-      if ((rc = time_cycles(m->stream, cycles_per_variant, one, ms))) return rc;
-      if (v == 0 || ms < best_ms) { best = v; best_ms = ms; }
-    }
-    if ((rc = or_model_set_variant(m, f, best))) return rc;
-  }
+  auto trial = [&](int h, int q, float &ms) -> int {
+    m->var_h = h;
+    m->var_q = q;
+    const LaunchSet L = model_set(m);
+    auto one = [&]() -> int {
+      const int p = (int)(m->parity & 1);
+      int r = (m->prec == OR_PREC_FP64) ? launch_cycle<double, double>(m->stream, L, p, nullptr, nullptr)
+                                        : launch_cycle<float, float>(m->stream, L, p, nullptr, nullptr);
+      m->parity ^= 1;
+      return r;
+    };
+    return time_cycles(m->stream, cycles_per_variant, one, ms);
+  };
+  int best[2];
+  rc = tune_variants(m->prec == OR_PREC_FP64, m->neh > 0, m->neq > 0, trial, best);
+  m->var_h = best[0];
+  m->var_q = best[1];
+  if (rc) return rc;
   chosen[0] = m->var_h;
   chosen[1] = m->var_q;
   return OR_OK;
@@ -3674,26 +3742,18 @@ int or_batch_autotune(or_batch *b, int32_t cycles_per_variant, int32_t chosen[4]
   if (!b || !chosen) return fail(OR_ERR_ARG, "null argument");
   if (cycles_per_variant < 1) return fail(OR_ERR_ARG, "cycles_per_variant must be >= 1");
   OR_HIP(hipSetDevice(b->device));
-  int rc;
-  for (int c = 0; c < 2; ++c)
-    for (int f = 0; f < 2; ++f) {
-      if ((rc = batch_rebuild(b))) return rc;
-      if (b->nt[c][f] == 0) continue;
-      int best = 0;
-      float best_ms = 0.f;
-      for (int v = 0; v < kVariants; ++v) {
-        b->var[c][f] = v;
-        b->dirty = true;
-        if ((rc = batch_rebuild(b))) return rc;
-        float ms = 0.f;
-        auto one = [&]() { return or_batch_run(b, 1); };
-        if ((rc = time_cycles(b->stream, cycles_per_variant, one, ms))) return rc;
-        if (v == 0 || ms < best_ms) { best = v; best_ms = ms; }
-      }
-      b->var[c][f] = best;
-      b->dirty = true;
-    }
-  if ((rc = batch_rebuild(b))) return rc;
+  int rc = batch_rebuild(b);
+  if (rc) return rc;
+  for (auto &v : b->var) v[0] = v[1] = 0;
+  for (int c = 0; c < 2; ++c) {
+    auto trial = [&](int h, int q, float &ms) -> int {
+      b->var[c][0] = h;
+      b->var[c][1] = q;
+      return time_cycles(b->stream, cycles_per_variant, [&]() { return or_batch_run(b, 1); }, ms);
+    };
+    rc = tune_variants(c == 0, b->nt[c][0] > 0, b->nt[c][1] > 0, trial, b->var[c]);
+    if (rc) return rc;
+  }
   for (int c = 0; c < 2; ++c)
     for (int f = 0; f < 2; ++f) chosen[2 * c + f] = b->var[c][f];
   return OR_OK;
