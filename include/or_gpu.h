@@ -14,6 +14,12 @@
  *                                       (scumu3p.F, cupdt3.F:967, asspar4.F:164-180)
  * The resident-model API takes 0-based indices (documented per call).
  *
+ * Memory kept between calls: the group and nodal drop-ins, uploads and read-backs go through
+ * page-locked host buffers, the nodal drop-in through a device workspace as well.  Up to 128 MiB of
+ * each stay allocated, idle, for the process's later calls from any thread (a larger one is freed
+ * after its call), until the process ends; idle ones are also freed when an allocation of this
+ * library finds no memory.  Transfers above 1 MiB use up to six threads while the call lasts.
+ *
  * Reference interfaces replaced (file:line in the OpenRadioss tree):
  *   or_model_*            the resident GPU handle of the shell offload module
  *                         (engine/source/elements/shell/coque/shell_gpu_mod.F90:279-715,

@@ -35,6 +35,7 @@
 #include "or_assembly.h"
 #include "or_hex.h"
 #include "or_q4.h"
+#include "or_staging.h"
 
 using namespace orgpu;
 
@@ -1575,12 +1576,43 @@ int make_q4_consts(const or_q4_params &p, Q4Consts &c) {
   return OR_OK;
 }
 
+#ifndef OR_ILP_TU
+// The buffers kept between calls (or_staging.h): allocating and freeing one costs more than a group's
+// whole call (2.0 ms with 15 of them, 0.05 ms now, of which the kernel is 0.02).
+struct HipMem {
+  static int alloc(int device, size_t bytes, void **p) {
+    const hipError_t e = device < 0 ? hipHostMalloc(p, bytes, hipHostMallocPortable | hipHostMallocMapped)
+                                    : hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError(); // reported here, not by the thread's next launch
+    return (int)e;
+  }
+  static void free(int device, void *p) { (void)(device < 0 ? hipHostFree(p) : hipFree(p)); }
+};
+typedef orstage::BufferPool<HipMem> StagePool;
+StagePool &stage_pool() {
+  static StagePool *pool = new StagePool; // outlives every static object
+  return *pool;
+}
+
+// hipMalloc on the current device; when memory runs out, once more without the idle workspaces.
+hipError_t device_alloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  int device = 0;
+  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && stage_pool().drop(device, 0)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 template <typename T> int dalloc(T **p, int64_t n, int64_t &acc) {
   if (n <= 0) { *p = nullptr; return OR_OK; }
-  OR_HIP(hipMalloc((void **)p, sizeof(T) * (size_t)n));
+  OR_HIP(device_alloc((void **)p, sizeof(T) * (size_t)n));
   acc += (int64_t)(sizeof(T) * (size_t)n);
   return OR_OK;
 }
+
+#endif // OR_ILP_TU
 
 } // namespace
 
@@ -1588,89 +1620,17 @@ template <typename T> int dalloc(T **p, int64_t n, int64_t &acc) {
 // ============================================================== staging
 namespace {
 
-// Page-locked host buffers (and device workspaces of the nodal drop-in) kept from one call to the
-// next: allocating and freeing one costs more than a group's whole call (2.0 ms with 15 of them,
-// 0.05 ms now, of which the kernel is 0.02).  A lease belongs to one call at a time; idle buffers
-// are kept up to kKeepBytes together (the oldest goes first) and freed at process end.
-class StagePool {
- public:
-  static constexpr size_t kKeepBytes = (size_t)128 << 20;
-  struct Buf {
-    void *p = nullptr;
-    size_t bytes = 0;
-    int device = -1; // -1: page-locked host memory
-  };
-  static StagePool &get() {
-    static StagePool *pool = new StagePool; // outlives every static object
-    return *pool;
-  }
-  hipError_t take(int device, size_t bytes, Buf &out) {
-    {
-      std::lock_guard<std::mutex> lock(m_);
-      size_t best = idle_.size();
-      for (size_t k = 0; k < idle_.size(); ++k)
-        if (idle_[k].device == device && idle_[k].bytes >= bytes && (best == idle_.size() || idle_[k].bytes < idle_[best].bytes))
-          best = k;
-      if (best < idle_.size()) {
-        out = idle_[best];
-        held_ -= out.bytes;
-        idle_.erase(idle_.begin() + (ptrdiff_t)best);
-        return hipSuccess;
-      }
-    }
-    out.device = device;
-    out.bytes = ((bytes + ((size_t)1 << 18) - 1) >> 18) << 18;
-    const hipError_t e = device < 0 ? hipHostMalloc(&out.p, out.bytes, hipHostMallocPortable | hipHostMallocMapped)
-                                    : hipMalloc(&out.p, out.bytes);
-    if (e != hipSuccess) out.p = nullptr;
-    return e;
-  }
-  void give(const Buf &b) {
-    if (!b.p) return;
-    std::vector<Buf> drop;
-    {
-      std::lock_guard<std::mutex> lock(m_);
-      if (!exit_) { // the handler runs before the HIP runtime's own, which was there first
-        exit_ = true;
-        std::atexit([] { get().clear(); });
-      }
-      idle_.push_back(b);
-      held_ += b.bytes;
-      while (held_ > kKeepBytes) {
-        drop.push_back(idle_.front());
-        held_ -= idle_.front().bytes;
-        idle_.erase(idle_.begin());
-      }
-    }
-    for (const Buf &d : drop) release(d);
-  }
-  void clear() {
-    std::vector<Buf> all;
-    {
-      std::lock_guard<std::mutex> lock(m_);
-      all.swap(idle_);
-      held_ = 0;
-    }
-    for (const Buf &b : all) release(b);
-  }
-
- private:
-  static void release(const Buf &b) {
-    if (b.p) (void)(b.device < 0 ? hipHostFree(b.p) : hipFree(b.p));
-  }
-  std::mutex m_;
-  std::vector<Buf> idle_; // oldest first
-  size_t held_ = 0;
-  bool exit_ = false;
-};
-
 struct Lease {
-  StagePool::Buf b;
+  StagePool::Buf b; // given back at the end of the scope
   Lease() = default;
   Lease(const Lease &) = delete;
   Lease &operator=(const Lease &) = delete;
-  ~Lease() { StagePool::get().give(b); }
-  hipError_t take(int device, size_t bytes) { return StagePool::get().take(device, bytes, b); }
+  ~Lease() {
+    static std::once_flag exit_handler; // runs before the HIP runtime's own, which is there by now
+    if (b.p) std::call_once(exit_handler, [] { (void)std::atexit([] { stage_pool().clear(); }); });
+    stage_pool().give(b);
+  }
+  hipError_t take(int device, size_t bytes) { return (hipError_t)stage_pool().take(device, bytes, b); }
   double *d() const { return (double *)b.p; }
 };
 
@@ -1984,7 +1944,7 @@ int or_model_create(or_model **out, int device, int64_t nn, int64_t ne_hex, int6
   const size_t ss = ssize(m);
   auto AS = [&](void **p, int64_t n) {
     if (rc != OR_OK || n <= 0) return;
-    if (hipMalloc(p, ss * (size_t)n) != hipSuccess) { rc = fail(OR_ERR_HIP, "hipMalloc state"); return; }
+    if (device_alloc(p, ss * (size_t)n) != hipSuccess) { rc = fail(OR_ERR_HIP, "hipMalloc state"); return; }
     m->bytes += (int64_t)(ss * (size_t)n);
   };
   A(&m->xv, 6 * nn);
@@ -2105,7 +2065,7 @@ int or_model_set_q4_params(or_model *m, const or_q4_params *p) {
   if (c.israte > 0 && m->neq > 0 && !m->qepsdip) {
     const size_t ss = ssize(m);
     OR_HIP(hipSetDevice(m->device));
-    OR_HIP(hipMalloc(&m->qepsdip, ss * (size_t)(m->npt * m->neq)));
+    OR_HIP(device_alloc(&m->qepsdip, ss * (size_t)(m->npt * m->neq)));
     OR_HIP(hipMemsetAsync(m->qepsdip, 0, ss * (size_t)(m->npt * m->neq), m->stream));
     OR_HIP(quiesce(m));
     m->bytes += (int64_t)(ss * (size_t)(m->npt * m->neq));
@@ -2150,7 +2110,7 @@ int or_model_upload_nodes(or_model *m, const double *x, const double *v, const d
   for (int64_t n = 0; code && n < nn && !imposed; ++n) imposed = (code[n] & (kIX | kIY | kIZ)) != 0;
   if (imposed && !m->wext) {
     OR_HIP(quiesce(m));
-    OR_HIP(hipMalloc((void **)&m->wext, sizeof(double) * 2 * (size_t)nn));
+    OR_HIP(device_alloc((void **)&m->wext, sizeof(double) * 2 * (size_t)nn));
     m->bytes += (int64_t)(sizeof(double) * 2 * nn);
     mark_changed(m);
   }
@@ -2407,9 +2367,9 @@ int or_model_upload_skyline(or_model *m, const int64_t *adsky, const int64_t *ia
     int32_t **frn = f == 0 ? &m->hfr_node : &m->qfr_node;
     uint16_t **frs = f == 0 ? &m->hfr_src : &m->qfr_src;
     const size_t nrow = ss * (size_t)(plan.nrest * W);
-    OR_HIP(hipMalloc(rows, nrow ? nrow : ss));
-    OR_HIP(hipMalloc((void **)frn, sizeof(int32_t) * (size_t)std::max<int64_t>(nfr, 1)));
-    OR_HIP(hipMalloc((void **)frs, sizeof(uint16_t) * orasm::kRunCap * (size_t)std::max<int64_t>(nfr, 1)));
+    OR_HIP(device_alloc(rows, nrow ? nrow : ss));
+    OR_HIP(device_alloc((void **)frn, sizeof(int32_t) * (size_t)std::max<int64_t>(nfr, 1)));
+    OR_HIP(device_alloc((void **)frs, sizeof(uint16_t) * orasm::kRunCap * (size_t)std::max<int64_t>(nfr, 1)));
     m->sky_bytes += (int64_t)(nrow + (4 + 2 * orasm::kRunCap) * (size_t)nfr);
     const std::vector<int32_t> &deg = f == 0 ? nh : nq;
     hipStream_t st = m->stream;
@@ -2700,8 +2660,8 @@ static int ensure_ctrl(or_model *m) {
     if (ne <= 0) return OR_OK;
     std::vector<int32_t> li((size_t)ne);
     for (int64_t s = 0; s < ne; ++s) li[(size_t)s] = perm.empty() ? (int32_t)s : perm[(size_t)s];
-    OR_HIP(hipMalloc((void **)dt, sizeof(double) * (size_t)ne));
-    OR_HIP(hipMalloc((void **)lidx, sizeof(int32_t) * (size_t)ne));
+    OR_HIP(device_alloc((void **)dt, sizeof(double) * (size_t)ne));
+    OR_HIP(device_alloc((void **)lidx, sizeof(int32_t) * (size_t)ne));
     OR_HIP(hipMemcpy(*lidx, li.data(), sizeof(int32_t) * (size_t)ne, hipMemcpyHostToDevice));
     m->bytes += (int64_t)(12 * ne);
     return OR_OK;
@@ -2709,7 +2669,7 @@ static int ensure_ctrl(or_model *m) {
   int rc = put(&m->dtel_h, &m->lidx_h, m->hperm, m->neh);
   if (rc == OR_OK) rc = put(&m->dtel_q, &m->lidx_q, m->qperm, m->neq);
   if (rc) return rc;
-  OR_HIP(hipMalloc((void **)&m->ctrl, 4 * sizeof(unsigned long long)));
+  OR_HIP(device_alloc((void **)&m->ctrl, 4 * sizeof(unsigned long long)));
   m->bytes += 32;
   mark_changed(m);
   return OR_OK;
@@ -2724,7 +2684,7 @@ int or_model_run_ecrit(or_model *m, or_ecrit *out) {
   OR_HIP(hipSetDevice(m->device));
   if (!m->ecrit) {
     OR_HIP(quiesce(m));
-    OR_HIP(hipMalloc((void **)&m->ecrit, sizeof(double) * 5 * (size_t)m->nn));
+    OR_HIP(device_alloc((void **)&m->ecrit, sizeof(double) * 5 * (size_t)m->nn));
     m->bytes += (int64_t)(sizeof(double) * 5 * m->nn);
     mark_changed(m);
   }
@@ -2822,26 +2782,26 @@ int or_model_th_setup(or_model *m, int64_t n_node, const int32_t *node, int64_t 
   for (void **p : {(void **)&m->th_slot, (void **)&m->th_hex, (void **)&m->th_q4, (void **)&m->th_buf})
     if (*p) { (void)hipFree(*p); *p = nullptr; }
   const int64_t words = 18 * n_node + 13 * n_hex + (12 + m->npt) * n_q4 + 1;
-  OR_HIP(hipMalloc((void **)&m->th_slot, sizeof(int32_t) * (size_t)m->nn));
+  OR_HIP(device_alloc((void **)&m->th_slot, sizeof(int32_t) * (size_t)m->nn));
   OR_HIP(hipMemcpy(m->th_slot, slot.data(), sizeof(int32_t) * (size_t)m->nn, hipMemcpyHostToDevice));
-  OR_HIP(hipMalloc((void **)&m->th_buf, sizeof(double) * (size_t)words));
+  OR_HIP(device_alloc((void **)&m->th_buf, sizeof(double) * (size_t)words));
   OR_HIP(hipMemset(m->th_buf, 0, sizeof(double) * (size_t)words));
   if (n_hex) {
-    OR_HIP(hipMalloc((void **)&m->th_hex, sizeof(int32_t) * (size_t)n_hex));
+    OR_HIP(device_alloc((void **)&m->th_hex, sizeof(int32_t) * (size_t)n_hex));
     OR_HIP(hipMemcpy(m->th_hex, hs.data(), sizeof(int32_t) * (size_t)n_hex, hipMemcpyHostToDevice));
   }
   if (n_q4) {
-    OR_HIP(hipMalloc((void **)&m->th_q4, sizeof(int32_t) * (size_t)n_q4));
+    OR_HIP(device_alloc((void **)&m->th_q4, sizeof(int32_t) * (size_t)n_q4));
     OR_HIP(hipMemcpy(m->th_q4, qs.data(), sizeof(int32_t) * (size_t)n_q4, hipMemcpyHostToDevice));
   }
   // EHOUR accumulates from the first setup on (a later setup keeps it)
   if (m->nt_h > 0 && !m->ehou_h) {
-    OR_HIP(hipMalloc((void **)&m->ehou_h, sizeof(double) * (size_t)m->nt_h));
+    OR_HIP(device_alloc((void **)&m->ehou_h, sizeof(double) * (size_t)m->nt_h));
     OR_HIP(hipMemset(m->ehou_h, 0, sizeof(double) * (size_t)m->nt_h));
     m->bytes += 8 * (int64_t)m->nt_h;
   }
   if (m->nt_q > 0 && !m->ehou_q) {
-    OR_HIP(hipMalloc((void **)&m->ehou_q, sizeof(double) * (size_t)m->nt_q));
+    OR_HIP(device_alloc((void **)&m->ehou_q, sizeof(double) * (size_t)m->nt_q));
     OR_HIP(hipMemset(m->ehou_q, 0, sizeof(double) * (size_t)m->nt_q));
     m->bytes += 8 * (int64_t)m->nt_q;
   }
@@ -3125,7 +3085,7 @@ struct Stage {
   }
   template <typename T> T *up(const T *h, size_t n) {
     T *d = nullptr;
-    if (e == hipSuccess) e = hipMalloc((void **)&d, sizeof(T) * (n ? n : 1));
+    if (e == hipSuccess) e = device_alloc((void **)&d, sizeof(T) * (n ? n : 1));
     ptrs.push_back(d);
     if (e == hipSuccess && h && n) e = hipMemcpy(d, h, sizeof(T) * n, hipMemcpyHostToDevice);
     return d;
@@ -3449,7 +3409,7 @@ int batch_rebuild(or_batch *b) {
     if (b->md) OR_HIP(hipFree(b->md));
     b->md = nullptr;
     b->md_cap = 0;
-    OR_HIP(hipMalloc((void **)&b->md, sizeof(ModelDev) * (size_t)ns));
+    OR_HIP(device_alloc((void **)&b->md, sizeof(ModelDev) * (size_t)ns));
     b->md_cap = ns;
   }
   std::vector<ModelDev> hd((size_t)ns);
@@ -3472,7 +3432,7 @@ int batch_rebuild(or_batch *b) {
         if (b->tiles[c][f]) OR_HIP(hipFree(b->tiles[c][f]));
         b->tiles[c][f] = nullptr;
         b->tcap[c][f] = 0;
-        OR_HIP(hipMalloc((void **)&b->tiles[c][f], sizeof(Tile) * (size_t)n));
+        OR_HIP(device_alloc((void **)&b->tiles[c][f], sizeof(Tile) * (size_t)n));
         b->tcap[c][f] = n;
       }
       if (n > 0) OR_HIP(hipMemcpy(b->tiles[c][f], tl[c][f].data(), sizeof(Tile) * (size_t)n, hipMemcpyHostToDevice));
