@@ -1666,48 +1666,33 @@ class Chunks {
     for (const Chunk &c : c_) total += c.bytes;
     // a thread costs some 30 us to start, the time of 0.3 MB
     const int nt = (int)std::min<size_t>({(size_t)kThreads, c_.size(), 1 + (total >> 20)});
-    next_ = 0;
-    err_ = hipSuccess;
-    std::vector<std::thread> team;
-    for (int t = 1; t < nt; ++t) {
-      try {
-        team.emplace_back([=] { work(device, st); });
-      } catch (const std::exception &) {
-        break; // no thread to be had: those that run take all the chunks
-      }
-    }
-    work(device, st);
-    for (std::thread &t : team) t.join();
+    const int e = orstage::run_team(nt, c_.size(), [&] { return Worker{c_, device, st}; });
     c_.clear();
-    return err_;
+    return (hipError_t)e;
   }
 
  private:
-  template <typename S> static void permuted(const Chunk &c, size_t n, S *out) {
-    const double *src = (const double *)c.host;
-    int64_t k = c.i0 / c.ne, s = c.i0 - k * c.ne;
-    for (size_t j = 0; j < n; ++j) {
-      out[j] = (S)src[k * c.ne + c.slot[s]];
-      if (++s == c.ne) { s = 0; ++k; }
-    }
-  }
-  void work(int device, hipStream_t st) {
-    Lease buf;
+  // One thread's buffer and event.
+  struct Worker {
+    const std::vector<Chunk> &chunks;
+    int device;
+    hipStream_t st;
+    Lease buf{};
     hipEvent_t ev = nullptr;
-    hipError_t e = hipSetDevice(device);
-    if (e == hipSuccess) e = buf.take(-1, 8 * kChunk);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     bool pending = false; // the buffer's last upload may still be read
-    while (e == hipSuccess) {
-      Chunk c;
-      {
-        std::lock_guard<std::mutex> lock(m_);
-        if (err_ != hipSuccess || next_ >= c_.size()) break;
-        c = c_[next_++];
-      }
+
+    int begin() {
+      hipError_t e = hipSetDevice(device);
+      if (e == hipSuccess) e = buf.take(-1, 8 * kChunk);
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+      return (int)e;
+    }
+    int item(size_t index) {
+      const Chunk &c = chunks[index];
+      hipError_t e = hipSuccess;
       if (pending) e = hipEventSynchronize(ev);
       pending = false;
-      if (e != hipSuccess) break;
+      if (e != hipSuccess) return (int)e;
       if (c.kind == Chunk::kUp || c.kind == Chunk::kUpElem64 || c.kind == Chunk::kUpElem32) {
         const size_t n = c.bytes / 8;
         size_t b = c.bytes, at = 0;
@@ -1717,7 +1702,7 @@ class Chunks {
         e = hipMemcpyAsync((char *)c.dev + at, buf.b.p, b, hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = hipEventRecord(ev, st);
         pending = e == hipSuccess;
-        continue;
+        return (int)e;
       }
       const int64_t n = (int64_t)(c.bytes / 8);
       const dim3 g((unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 512));
@@ -1732,23 +1717,30 @@ class Chunks {
       if (e == hipSuccess) e = hipEventRecord(ev, st);
       if (e == hipSuccess) e = hipEventSynchronize(ev);
       if (e == hipSuccess) std::memcpy(c.host, buf.b.p, c.bytes);
+      return (int)e;
     }
-    if (pending) {
-      const hipError_t f = hipEventSynchronize(ev);
-      if (e == hipSuccess) e = f;
-    } else if (e != hipSuccess) {
-      (void)hipStreamSynchronize(st); // nothing of this call may still use the buffer
+    int end(int e) { // nothing of this call may still use the buffer
+      if (pending) {
+        const hipError_t f = hipEventSynchronize(ev);
+        if (!e) e = (int)f;
+      } else if (e) {
+        (void)hipStreamSynchronize(st);
+      }
+      return e;
     }
-    if (ev) (void)hipEventDestroy(ev);
-    if (e != hipSuccess) {
-      std::lock_guard<std::mutex> lock(m_);
-      if (err_ == hipSuccess) err_ = e;
+    ~Worker() {
+      if (ev) (void)hipEventDestroy(ev);
+    }
+  };
+  template <typename S> static void permuted(const Chunk &c, size_t n, S *out) {
+    const double *src = (const double *)c.host;
+    int64_t k = c.i0 / c.ne, s = c.i0 - k * c.ne;
+    for (size_t j = 0; j < n; ++j) {
+      out[j] = (S)src[k * c.ne + c.slot[s]];
+      if (++s == c.ne) { s = 0; ++k; }
     }
   }
   std::vector<Chunk> c_;
-  size_t next_ = 0;
-  std::mutex m_;
-  hipError_t err_ = hipSuccess;
 };
 
 } // namespace

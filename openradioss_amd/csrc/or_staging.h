@@ -1,8 +1,10 @@
-// Buffers kept between calls, without HIP: the allocator is a template argument (or_capi.hip's, or a
-// counting one in the CPU test).
+// Buffers kept between calls and the threads that share a transfer, without HIP: the allocator and the
+// worker are template arguments (or_capi.hip's, or the CPU test's).
 #pragma once
 #include <cstddef>
+#include <exception>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 namespace orstage {
@@ -102,5 +104,42 @@ template <class Mem> class BufferPool {
   std::vector<Buf> idle_; // oldest first
   size_t held_[2] = {0, 0};
 };
+
+// Items 0..n-1, taken in turn by the calling thread and up to nt - 1 helpers, each with a worker of its own
+// from make(): begin() and end(error) around its items, 0 for success.  A helper that cannot be
+// started or cannot begin (no buffer to be had) leaves its share to the others; only the caller's
+// begin, an item or an end that fails ends the whole with its error.
+template <class Make> int run_team(int nt, size_t n, const Make &make) {
+  std::mutex m;
+  size_t next = 0;
+  int err = 0;
+  auto work = [&](bool helper) {
+    auto w = make();
+    int e = w.begin();
+    if (e && helper) return;
+    while (!e) {
+      size_t k;
+      {
+        std::lock_guard<std::mutex> lock(m);
+        if (err || next >= n) break;
+        k = next++;
+      }
+      e = w.item(k);
+    }
+    e = w.end(e);
+    if (e) {
+      std::lock_guard<std::mutex> lock(m);
+      if (!err) err = e;
+    }
+  };
+  std::vector<std::thread> team;
+  try {
+    for (int t = 1; t < nt; ++t) team.emplace_back(work, true);
+  } catch (const std::exception &) { // no thread to be had
+  }
+  work(false);
+  for (std::thread &t : team) t.join();
+  return err;
+}
 
 } // namespace orstage

@@ -138,3 +138,51 @@ extern "C" int pool_threads(int nthreads, int rounds) {
   CHECK(g_live == 0 && g_bytes[0] == 0 && g_bytes[1] == 0 && g_bytes[2] == 0);
   return 0;
 }
+
+namespace {
+// A worker that counts; helpers are known by their thread.
+struct Counter {
+  std::atomic<int> *done, *begun, *ended;
+  std::thread::id caller;
+  int helper_fails, caller_fails, item_fails; // item_fails: from this item on
+  int begin() {
+    const bool helper = std::this_thread::get_id() != caller;
+    if (helper ? helper_fails : caller_fails) return helper ? helper_fails : caller_fails;
+    ++*begun;
+    return 0;
+  }
+  int item(size_t k) {
+    if ((int)k >= item_fails) return 7;
+    std::this_thread::yield();
+    ++done[k];
+    return 0;
+  }
+  int end(int e) { ++*ended; return e; }
+};
+} // namespace
+
+extern "C" int team_takes_every_item_once(int nt, int n) {
+  for (int helpers_fail = 0; helpers_fail < 2; ++helpers_fail) {
+    std::vector<std::atomic<int>> done((size_t)n);
+    std::atomic<int> begun{0}, ended{0};
+    const auto me = std::this_thread::get_id();
+    const int e = orstage::run_team(nt, (size_t)n, [&] {
+      return Counter{done.data(), &begun, &ended, me, helpers_fail ? 5 : 0, 0, n};
+    });
+    CHECK(e == 0); // also where no helper gets its buffer
+    for (auto &d : done) CHECK(d == 1);
+    CHECK(begun == ended && begun == (helpers_fail ? 1 : (nt > 0 ? nt : 1)));
+  }
+  return 0;
+}
+
+extern "C" int team_reports_errors() {
+  std::vector<std::atomic<int>> done(100);
+  std::atomic<int> begun{0}, ended{0};
+  const auto me = std::this_thread::get_id();
+  CHECK(orstage::run_team(1, 100, [&] { return Counter{done.data(), &begun, &ended, me, 0, 3, 100}; }) == 3);
+  for (auto &d : done) CHECK(d == 0);
+  CHECK(orstage::run_team(4, 100, [&] { return Counter{done.data(), &begun, &ended, me, 0, 0, 40}; }) == 7);
+  for (int k = 0; k < 100; ++k) CHECK(done[(size_t)k] == (k < 40 ? 1 : 0)); // taken in order, none after the failure
+  return 0;
+}

@@ -1,6 +1,7 @@
 """The buffers that calls keep (openradioss_amd/csrc/or_staging.h) on the CPU, with a counting allocator:
 large workspaces push out no host buffers, limits hold, memory running out gives the idle buffers
-up, and a buffer belongs to one call at a time.  Built here from tests/stage_check.cpp with g++."""
+up, and a buffer belongs to one call at a time.  The
+threads that share a transfer: a helper without a buffer leaves its share to the others.  Built here from tests/stage_check.cpp with g++."""
 import ctypes as C
 import os
 import subprocess
@@ -27,4 +28,15 @@ def test_pool(check, case):
 
 def test_pool_with_threads(check):
     line = check.pool_threads(8, 2000)
+    assert line == 0, f"stage_check.cpp:{line}"
+
+
+@pytest.mark.parametrize("threads,items", [(1, 0), (1, 3), (6, 1), (6, 5), (6, 400)])
+def test_team_takes_every_item_once(check, threads, items):
+    line = check.team_takes_every_item_once(threads, items)
+    assert line == 0, f"stage_check.cpp:{line}"
+
+
+def test_team_reports_errors(check):
+    line = check.team_reports_errors()
     assert line == 0, f"stage_check.cpp:{line}"
