@@ -1157,8 +1157,15 @@ __global__ __launch_bounds__(kBlock) void k_energy_final(const double *partial, 
 }
 
 template <typename T> __global__ __launch_bounds__(kBlock) void k_fill(T *p, int64_t n, T v) {
-  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (j < n) p[j] = v;
+  for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < n; j += (int64_t)gridDim.x * kBlock) p[j] = v;
+}
+// A launch holds fewer than 2^32 threads, a state array of ten points more values than that from 86
+// million shells on: 16,384 blocks at most, which fill the chip eight times over.
+template <typename T> hipError_t fill(hipStream_t st, T *p, int64_t n, T v) {
+  if (n <= 0) return hipSuccess;
+  const unsigned g = (unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 16384);
+  hipLaunchKernelGGL(k_fill<T>, dim3(g), dim3(kBlock), 0, st, p, n, v);
+  return hipGetLastError();
 }
 
 // The element that controls the time step of an output cycle, as MQVISCB and CDT3 name it
@@ -2132,10 +2139,8 @@ static int put_state(or_model *m, Chunks &io, void *dst, const double *src, int6
               (int64_t)perm.size(), perm.data());
     return OR_OK;
   }
-  const unsigned g = (unsigned)((n + kBlock - 1) / kBlock);
-  if (m->prec == OR_PREC_FP64) hipLaunchKernelGGL(k_fill<double>, dim3(g), dim3(kBlock), 0, m->stream, (double *)dst, n, dflt);
-  else hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kBlock), 0, m->stream, (float *)dst, n, (float)dflt);
-  OR_HIP(hipGetLastError());
+  if (m->prec == OR_PREC_FP64) OR_HIP(fill(m->stream, (double *)dst, n, dflt));
+  else OR_HIP(fill(m->stream, (float *)dst, n, (float)dflt));
   return OR_OK;
 }
 // An element array of the caller's order, read back by the export kernels.
@@ -2683,14 +2688,8 @@ int or_model_run_ecrit(or_model *m, or_ecrit *out) {
   int rc = ensure_ctrl(m);
   if (rc) return rc;
   // candidates of elements that cannot control the step (and of a stopped model) stay EP06
-  auto fill_ep06 = [&](double *p, int64_t n) -> int {
-    if (n > 0)
-      hipLaunchKernelGGL(k_fill<double>, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, m->stream, p, n,
-                         kEP06);
-    OR_HIP(hipGetLastError());
-    return OR_OK;
-  };
-  if ((rc = fill_ep06(m->dtel_h, m->neh)) || (rc = fill_ep06(m->dtel_q, m->neq))) return rc;
+  OR_HIP(fill(m->stream, m->dtel_h, m->neh, kEP06));
+  OR_HIP(fill(m->stream, m->dtel_q, m->neq, kEP06));
   rc = refresh_dev(m);
   if (rc) return rc;
   const LaunchSet L = model_set(m);
