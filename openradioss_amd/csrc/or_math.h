@@ -26,7 +26,8 @@
 // the low word in plain double, fused multiply-adds) and keeps its result only when every
 // value within kFastErr of it rounds to the same double (Ziv's rounding test, ACM TOMS
 // 17(3), 1991); the double-double value lies within that distance, so both give the same
-// bits.  The test fails for about 1 argument in 10,000, which takes the double-double path.
+// bits.  Over the path's ranges the test fails for 1 argument in 8,000 (exp, pow) or 41,000 (log), which
+// takes the double-double path.
 // What it is for: a plastic shell point calls log and exp five times in one dependent
 // chain, and a wave's chain, not the issue rate, bounds the shell kernel.
 #pragma once
@@ -225,8 +226,10 @@ __host__ __device__ __forceinline__ bool try_pow_from_log(double y, dd l, double
   if (!(y >= -1.0 && y <= 1.0) || y == 0.0 || !(zh > -700.0 && zh < 700.0)) return false;
   return exp_fast(zh, fma(y, l.hi, -zh) + y * l.lo, res, tab);
 }
+// FAST, of the functions below: the short evaluation is tried first.  The host build keeps to the
+// double-double path unless it asks for the device's.
 #if defined(__HIP_DEVICE_COMPILE__)
-constexpr bool kTryFast = true; // the host build keeps to the double-double path
+constexpr bool kTryFast = true;
 #else
 constexpr bool kTryFast = false;
 #endif
@@ -235,32 +238,32 @@ constexpr bool kTryFast = false;
 constexpr double kMinNormal = 0x1.0p-1022;
 constexpr double kMaxFinite = 0x1.fffffffffffffp+1023;
 
-template <class T = GlobalTab>
+template <class T = GlobalTab, bool FAST = kTryFast>
 __host__ __device__ inline double or_log(double x, const T tab = T{}) {
   if (!(x >= kMinNormal && x <= kMaxFinite)) return log(x);
   double f;
-  if (kTryFast && try_log(x, f, tab)) return f;
+  if (FAST && try_log(x, f, tab)) return f;
   // the rare path reads the constant arrays: through the shells' copy in LDS it costs them registers
   // that spill (28 bytes a lane)
   dd l = log_dd(x);
   return l.hi + l.lo;
 }
 
-template <class T = GlobalTab>
+template <class T = GlobalTab, bool FAST = kTryFast>
 __host__ __device__ inline double or_exp(double z, const T tab = T{}) {
   if (!(z > -708.0 && z < 708.0)) return exp(z);
   double f;
-  if (kTryFast && exp_fast(z, 0.0, f, tab)) return f;
+  if (FAST && exp_fast(z, 0.0, f, tab)) return f;
   return exp_dd(z, 0.0, tab);
 }
 
-template <class T = GlobalTab>
+template <class T = GlobalTab, bool FAST = kTryFast>
 __host__ __device__ inline double or_pow(double x, double y, const T tab = T{}) {
   if (x == 0.0 && y > 0.0) return 0.0;
   if (y == 0.0 || x == 1.0) return 1.0;
   if (!(x >= kMinNormal && x <= kMaxFinite) || !(y >= -kMaxFinite && y <= kMaxFinite)) return pow(x, y);
   double f;
-  if (kTryFast && try_pow_from_log(y, log_fast(x, tab), f, tab)) return f;
+  if (FAST && try_pow_from_log(y, log_fast(x, tab), f, tab)) return f;
   dd l = log_dd(x, tab);
   dd z = two_prod(y, l.hi);
   z.lo = z.lo + y * l.lo;
@@ -281,15 +284,15 @@ __host__ __device__ inline double pow_from_log(double x, double y, dd l, const T
   if (!(z.hi > -708.0 && z.hi < 708.0)) return pow(x, y);
   return exp_dd(z.hi, z.lo, tab);
 }
-template <class T = GlobalTab>
+template <class T = GlobalTab, bool FAST = kTryFast>
 __host__ __device__ inline void or_pow2(double x, double y1, double y2, double &r1, double &r2,
                                         const T tab = T{}) {
   if (!(x >= kMinNormal && x <= kMaxFinite) || x == 1.0) {
-    r1 = or_pow(x, y1, tab);
-    r2 = or_pow(x, y2, tab);
+    r1 = or_pow<T, FAST>(x, y1, tab);
+    r2 = or_pow<T, FAST>(x, y2, tab);
     return;
   }
-  if (kTryFast) {
+  if (FAST) {
     const dd l = log_fast(x, tab);
     const bool ok1 = try_pow_from_log(y1, l, r1, tab), ok2 = try_pow_from_log(y2, l, r2, tab);
     if (ok1 && ok2) return;

@@ -123,3 +123,34 @@ int64_t or_cr_pow2_check(int64_t n, uint64_t seed) {
   return bad;
 }
 }
+
+extern "C" {
+// The device's short evaluations of function fn (0 log, 1 exp, 2 pow) on this side: accepted[i] is 1
+// where the rounding test keeps the value out[i].
+void or_short_eval(int fn, int64_t n, const double *x, const double *y, double *out, uint8_t *accepted) {
+  for (int64_t i = 0; i < n; ++i)
+    accepted[i] = fn == 0   ? ormath::try_log(x[i], out[i])
+                  : fn == 1 ? ormath::exp_fast(x[i], 0.0, out[i])
+                            : ormath::try_pow_from_log(y[i], ormath::log_fast(x[i]), out[i]);
+}
+// The functions as the device runs them: the short evaluation first, the double-double path where it is
+// rejected.
+void or_device_eval(int fn, int64_t n, const double *x, const double *y, double *out) {
+  using ormath::GlobalTab;
+  for (int64_t i = 0; i < n; ++i)
+    out[i] = fn == 0   ? ormath::or_log<GlobalTab, true>(x[i])
+             : fn == 1 ? ormath::or_exp<GlobalTab, true>(x[i])
+                       : ormath::or_pow<GlobalTab, true>(x[i], y[i]);
+}
+// or_pow2 as the device runs it against the double-double powers; returns the mismatching pairs.
+int64_t or_device_pow2_check(int64_t n, const double *x, const double *y1, const double *y2) {
+  int64_t bad = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    double r1, r2;
+    ormath::or_pow2<ormath::GlobalTab, true>(x[i], y1[i], y2[i], r1, r2);
+    const double p1 = or_cr_pow(x[i], y1[i]), p2 = or_cr_pow(x[i], y2[i]);
+    bad += memcmp(&r1, &p1, 8) != 0 || memcmp(&r2, &p2, 8) != 0;
+  }
+  return bad;
+}
+}
