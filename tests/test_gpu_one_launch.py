@@ -60,3 +60,22 @@ def test_batch(forms, gpu_lib):
         ref = separate(m, p)
         ref.run(g.time_state().ncycle if k == 1 else 40)
         same(g, ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "split"])
+@pytest.mark.parametrize("k", [0, 1])
+def test_time_history(k, precision, gpu_lib):
+    """The instantiations that keep EHOUR (hourglass energy of each tile) and an output cycle's candidates."""
+    print(f"case: mixed model {k} with a time history, {precision}, 30 cycles and 3 records", flush=True)
+    m = models()[k]
+    a, b = E.GpuModel(m, precision=precision), separate(m, precision)
+    for g in (a, b):
+        g.th_setup(range(0, m.nn, 7), range(0, m.ne_hex, 5), range(0, m.ne_q4, 3))
+    for _ in range(3):
+        a.run(9)
+        b.run(9)
+        ra, rb = a.run_th(), b.run_th()
+        assert ra["ehour"] != 0.0
+        assert all(np.array_equal(ra[n], rb[n]) for n in ra)
+        assert a.ehour() == b.ehour() == ra["ehour"]
+    same(a, b)
