@@ -304,8 +304,9 @@ int or_batch_active(or_batch *b, int32_t *nactive);
  * FP64, and the split form's hexes with v = 1.  Every workgroup is one tile of 256 elements.
  * All variants compute bit-identical results.  Families of default variants share one launch.
  * The autotuners time 4 * cycles_per_variant real cycles a family (the models advance
- * meanwhile), the joint launch among the candidates, and keep the fastest; the default unless
- * another is 2 % faster: chosen[family] for a model, chosen[2*precision + family] for a batch. */
+ * meanwhile), the joint launch among the candidates, and keep the fastest (in place of a joint
+ * launch, one that is 1 % faster): chosen[family] for a model, chosen[2*precision + family] for
+ * a batch. */
 int or_model_set_variant(or_model *m, int family, int variant);
 int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]);
 int or_batch_autotune(or_batch *b, int32_t cycles_per_variant, int32_t chosen[4]);

@@ -3631,9 +3631,9 @@ template <typename F> int time_cycles(hipStream_t st, int ncycles, F launch, flo
 // cycles with variants h and q.  The default pair, whose families share a launch, is measured
 // against pairs with a launch each: hexes' other variants, shells' with the best of those, the default
 // hexes with the best shells.  kVariants trials a family in all; those left over repeat the default and
-// the best other pair, whose shortest times count.  Another pair is taken only when it is 2 %
-// faster, which is what two measurements of one pair differ by.
-template <typename F> int tune_variants(bool fp64, bool has_hex, bool has_q4, F trial, int best[2]) {
+// the best other pair, whose shortest times count.  Where a joint launch is at stake another pair is
+// taken only when it is 1 % faster, which is what two measurements of one pair differ by.
+template <typename F> int tune_variants(bool fp64, bool has_hex, bool has_q4, bool joint, F trial, int best[2]) {
   constexpr float kNone = 1.0e30f;
   float t[kVariants][kVariants];
   for (auto &row : t) std::fill(std::begin(row), std::end(row), kNone);
@@ -3670,7 +3670,7 @@ template <typename F> int tune_variants(bool fp64, bool has_hex, bool has_q4, F 
     run(h, q);
   }
   const float ms = fastest_other(h, q);
-  const bool take = rc == OR_OK && ms < 0.98f * t[0][0];
+  const bool take = rc == OR_OK && ms < (joint ? 0.99f : 1.0f) * t[0][0];
   best[0] = take ? h : 0;
   best[1] = take ? q : 0;
   return rc;
@@ -3711,7 +3711,7 @@ int or_model_autotune(or_model *m, int32_t cycles_per_variant, int32_t chosen[2]
     return time_cycles(m->stream, cycles_per_variant, one, ms);
   };
   int best[2];
-  rc = tune_variants(m->prec == OR_PREC_FP64, m->neh > 0, m->neq > 0, trial, best);
+  rc = tune_variants(m->prec == OR_PREC_FP64, m->neh > 0, m->neq > 0, m->neh > 0 && m->neq > 0, trial, best);
   m->var_h = best[0];
   m->var_q = best[1];
   if (rc) return rc;
@@ -3733,7 +3733,9 @@ int or_batch_autotune(or_batch *b, int32_t cycles_per_variant, int32_t chosen[4]
       b->var[c][1] = q;
       return time_cycles(b->stream, cycles_per_variant, [&]() { return or_batch_run(b, 1); }, ms);
     };
-    rc = tune_variants(c == 0, b->nt[c][0] > 0, b->nt[c][1] > 0, trial, b->var[c]);
+    const bool hexes = b->nt[c][0] > 0, shells = b->nt[c][1] > 0;
+    const bool joint = (hexes && shells) || (b->nt[0][2] > 0 && b->nt[1][2] > 0);
+    rc = tune_variants(c == 0, hexes, shells, joint, trial, b->var[c]);
     if (rc) return rc;
   }
   for (int c = 0; c < 2; ++c)
