@@ -2584,9 +2584,10 @@ static LaunchSet model_set(const or_model *m) {
 
 // A set's element kernels run in one launch (k_elements) when both families are there, their
 // variants are the default one and nobody asked for the families' own times: the tiles of one
-// family fill the compute units that the other leaves idle.  Against one launch each: 13,824
-// hexes + 2,304 shells 20.7 us a cycle (29.8), 512,000 + 160,000 141.0 (151.2; split form 93.9 and
-// 104.4), a batch of 12 bars and tubes in both forms 47.0 (103.2).
+// family fill the compute units that the other leaves idle.  Against one launch each, us a cycle: 13,824
+// hexes + 2,304 shells 19.8 (29.8), 512,000 + 160,000 137 (151; split form 95 and 102), 4,096,000 +
+// 1,000,000 1,000 (1,027; 740 and 731, where the tuner finds the separate launches), a batch of 12 bars and
+// tubes in both forms 47.0 (103.2).
 static bool one_launch(const LaunchSet &L) { return L.nth > 0 && L.ntq > 0 && L.vh == 0 && L.vq == 0; }
 
 // Which form of the node update a launch of nb blocks takes.  A small model's update is a chain of
